@@ -11,6 +11,7 @@
 //             rounding after each add, then + sh          fused_int4.py:244 (index_add_),
 //                                                          transformers/.../modeling_qwen3_5_moe.py:796
 // The shared expert is one more group (id E) whose rows are all T tokens in order.
+#include <math.h>
 #include <stdlib.h>
 #include <string.h>
 #include <type_traits>
@@ -44,11 +45,11 @@ __device__ __forceinline__ bool ids_aligned(const int32_t* ids32, const int64_t*
 
 // ---------------------------------------------------------------- dispatch
 // One block of 1024 threads: per-expert counts, offsets, M-chunk schedule, inv := -1, and
-// (desc non-null) one descriptor per M-chunk: {group, rows, first row in group order, 0}.
+// (desc non-null) one descriptor per M-chunk of bm rows: {group, rows, first row in group order, 0}.
 __global__ __launch_bounds__(1024) void k_dispatch_count(const int32_t* ids32, const int64_t* ids64, int T, int k,
                                                          int E, int shared_rows, int32_t* offsets,
                                                          int32_t* tile_start, int32_t* inv, uint32_t* err,
-                                                         int4* desc) {
+                                                         int4* desc, int bm) {
   __shared__ int cnt[1024];
   const int tid = threadIdx.x;
   for (int e = tid; e < 1024; e += 1024) cnt[e] = 0;
@@ -85,7 +86,7 @@ __global__ __launch_bounds__(1024) void k_dispatch_count(const int32_t* ids32, c
   __syncthreads();
   // Inclusive Hillis-Steele scans of counts and M-chunks (groups 0..E-1, then the shared group).
   const int c = tid < E ? cnt[tid] : 0;
-  int ch = tid < E ? (c + kBM - 1) / kBM : (tid == E ? (shared_rows + kBM - 1) / kBM : 0);
+  int ch = tid < E ? (c + bm - 1) / bm : (tid == E ? (shared_rows + bm - 1) / bm : 0);
   __shared__ int sc[1024], sk[1025];
   sc[tid] = c;
   sk[tid] = ch;
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(1024) void k_dispatch_count(const int32_t* ids32, c
   if (tid == 0) { offsets[0] = 0; tile_start[0] = 0; }
   if (tid <= E) tile_start[tid + 1] = sk[tid];
   if (!desc) return;
-  // M-chunk mt of group g (sk[g - 1] <= mt < sk[g]): rows r0 = (mt - sk[g - 1]) kBM onwards.
+  // M-chunk mt of group g (sk[g - 1] <= mt < sk[g]): rows r0 = (mt - sk[g - 1]) bm onwards.
   const int n_groups = shared_rows > 0 ? E + 1 : E;
   const int n_chunks = sk[n_groups - 1];
   for (int mt = tid; mt < n_chunks; mt += 1024) {
@@ -113,10 +114,10 @@ __global__ __launch_bounds__(1024) void k_dispatch_count(const int32_t* ids32, c
       if (sk[mid] > mt) hi = mid; else lo = mid + 1;
     }
     const int g = lo;
-    const int r0 = (mt - (g ? sk[g - 1] : 0)) * kBM;
+    const int r0 = (mt - (g ? sk[g - 1] : 0)) * bm;
     const int rows = g < E ? cnt[g] : shared_rows;
     const int first = g < E ? (g ? sc[g - 1] : 0) : 0;
-    desc[mt] = int4{g, min(kBM, rows - r0), first + r0, 0};
+    desc[mt] = int4{g, min(bm, rows - r0), first + r0, 0};
   }
 }
 
@@ -1011,26 +1012,34 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_p(GemmParams p) {
 //   slots requested kWA stages ahead; the slot is a run-time index (stage % kWAS).
 // Iteration g: request A stage g + kWA; wait for weight stage g; its registers to the region;
 // request weight stage g + kWB into them; 40 MFMAs; wait for A stage g + 1; barrier.
-// K: a multiple of 4 stages (256) and at least 8 stages (the next tile's perm words, requested
-// after a tile's epilogue, are used before its last cycle, 4 stage waits later).
+// K: a multiple of WB stages and at least 2 WB (the next tile's perm words, requested
+// after a tile's epilogue, are used before its last cycle, WB stage waits later).
+// MB: 16-row token blocks per tile (10: 160-row chunks; 4 and 2 for smaller groups, whose padding
+// would otherwise be read and multiplied).
 // WB: weight stages in registers (the unrolled cycle; 4, or 5 where K / 64 is a multiple of
 // 5), A stages requested as far ahead (every request past a tile's end falls in its last
 // cycle), WB + 1 A ring slots.
 constexpr int kWBLoads = 2 * kPNB;            // weight loads per wave per stage (8 rows each)
 constexpr int kWReg = 16 * kPNB * 8;          // u32x4 per wave region (32 rows x 128 B)
-constexpr int kWOps = kPLoads + kWBLoads;     // vector memory operations per stage
 
-template <bool UP, int WB>
+template <bool UP, int WB, int MB>
 __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
   constexpr int kWB = WB, kWA = WB, kWAS = WB + 1;
-  static_assert(kWBLoads + (kWA - 1) * kWOps < 64 && (kWB - 1) * kWOps + kPLoads < 64, "vmcnt range");
-  static_assert((kWAS * kPSlot + kPW * kWReg) * 16 <= 160 * 1024, "LDS");
-  __shared__ u32x4 lA[kWAS * kPSlot];
+  constexpr int kSlot = MB * 16 * 8;             // u32x4 per A slot (16 MB rows x 128 B)
+  constexpr int kALoads = (2 * MB + kPW - 1) / kPW;   // A loads per wave per stage
+  constexpr int kWOps = kALoads + kWBLoads;      // vector memory operations per stage
+  static_assert(kWBLoads + (kWA - 1) * kWOps < 64 && (kWB - 1) * kWOps + kALoads < 64, "vmcnt range");
+  static_assert((kWAS * kSlot + kPW * kWReg) * 16 <= 160 * 1024, "LDS");
+  __shared__ u32x4 lA[kWAS * kSlot];
   __shared__ u32x4 lB[kPW * kWReg];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int K = p.K;
   u32x4* const reg = lB + wid * kWReg;
+  // The stage's 8-row parts are loads 0 .. 2 MB - 1 over the waves; a wave whose load index lies
+  // past them repeats an earlier part (the same bytes to the same place).
+  auto a_part = [](int x) { return MB == 1 ? (x & 1) : x < 2 * MB ? x : x - kPW / 2; };
+  static_assert(MB == 1 || (2 * MB) % kPW == 0 || (2 * MB) % kPW == kPW / 2, "repeats are earlier parts");
 
   const int c_lo = sload1(p.tile_start + p.group_lo);
   const int c_hi = sload1(p.tile_start + p.group_hi);
@@ -1078,11 +1087,11 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
   // repeating 16..19); weights: load 2 nb + h covers rows 16 nb + 8 h + lane / 8 of the
   // wave's two blocks, bytes 16 (lane % 8).
   const int lrow = lane & 15;
-  int a_row[kPLoads];
+  int a_row[kALoads];
 #pragma unroll
-  for (int j = 0; j < kPLoads; ++j) {
+  for (int j = 0; j < kALoads; ++j) {
     const int x = wid + kPW * j;
-    a_row[j] = 8 * (x < kBM / 8 ? x : x - kPW / 2) + (lane >> 3);
+    a_row[j] = 8 * (a_part(x)) + (lane >> 3);
   }
   const int a_col = 8 * ((lane & 7) ^ (lane >> 3));
   const int rd0 = lrow * 8 + ((lane >> 4) ^ (lrow & 7));          // fragment chunk, k 0..31
@@ -1092,10 +1101,10 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) b_off[h] = (uint32_t)(((8 * h + (lane >> 3)) * K + (lane & 7) * 8) * 2);
 
-  f32x4 acc[kPMB][kPNB];
+  f32x4 acc[MB][kPNB];
   auto zero_acc = [&]() {
 #pragma unroll
-    for (int i = 0; i < kPMB; ++i)
+    for (int i = 0; i < MB; ++i)
 #pragma unroll
       for (int nb = 0; nb < kPNB; ++nb) acc[i][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
   };
@@ -1103,19 +1112,19 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
 
   u32x4 breg[kWB][kWBLoads];
   const int nk = K / kBK;   // a multiple of kWB, at least 2 kWB
-  uint32_t a_off_cur[kPLoads], a_off_nxt[kPLoads];
-  uint32_t pv_cur[kPLoads], pv_nxt[kPLoads];
-  // Always kPLoads loads (tiles without a gather read perm[0]): the waits count them.
+  uint32_t a_off_cur[kALoads], a_off_nxt[kALoads];
+  uint32_t pv_cur[kALoads], pv_nxt[kALoads];
+  // Always kALoads loads (tiles without a gather read perm[0]): the waits count them.
   auto fetch_perm = [&](uint32_t* pv, const PTile& t) {
     const int32_t* pp = p.perm + (t.gather ? t.arow0 : 0);
 #pragma unroll
-    for (int j = 0; j < kPLoads; ++j) pv[j] = gld4(pp, t.gather ? (uint32_t)(min(a_row[j], t.m - 1) * 4) : 0u);
+    for (int j = 0; j < kALoads; ++j) pv[j] = gld4(pp, t.gather ? (uint32_t)(min(a_row[j], t.m - 1) * 4) : 0u);
   };
   auto a_offsets = [&](uint32_t* o, uint32_t* pv, const PTile& t) {
-    asm volatile("" : "+v"(pv[0]), "+v"(pv[1]), "+v"(pv[2]));
-    static_assert(kPLoads == 3, "three perm words per lane");
 #pragma unroll
-    for (int j = 0; j < kPLoads; ++j) {
+    for (int j = 0; j < kALoads; ++j) asm volatile("" : "+v"(pv[j]));
+#pragma unroll
+    for (int j = 0; j < kALoads; ++j) {
       const int row = t.gather ? (int)pv[j] / p.k : t.arow0 + min(a_row[j], t.m - 1);
       o[j] = (uint32_t)row * (uint32_t)(K * 2) + (uint32_t)(a_col * 2);
     }
@@ -1123,11 +1132,11 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
   auto gaddr = [](const void* base, size_t ofs) { return reinterpret_cast<const char*>(base) + ofs; };
   auto dma_a = [&](int slot, bool nx, int st) {
     const char* ta = gaddr(p.a, (size_t)st * kBK * 2);
-    u32x4* const s = lA + slot * kPSlot;
+    u32x4* const s = lA + slot * kSlot;
 #pragma unroll
-    for (int j = 0; j < kPLoads; ++j) {
+    for (int j = 0; j < kALoads; ++j) {
       const int x = wid + kPW * j;
-      gdma16(ta, nx ? a_off_nxt[j] : a_off_cur[j], s + (x < kBM / 8 ? x : x - kPW / 2) * 64);
+      gdma16(ta, nx ? a_off_nxt[j] : a_off_cur[j], s + (a_part(x)) * 64);
     }
   };
   auto load_b = [&](int bs, bool nx, int st) {
@@ -1142,12 +1151,16 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
   // Wait for weight stage bs (requested kWB - 1 iterations and one A group before, plus X
   // operations of an epilogue in between).  The registers pass through the asm, so nothing
   // reads them before the wait.
-  // Stores per thread in one epilogue (up: 2 passes x 3, down: 2 passes x 5); the first 4
-  // iterations of the next tile add them and the next tile's perm loads (kXH) to their waits.
-  constexpr int kEpiStores = UP ? 6 : 10;
-  constexpr int kXH = kEpiStores + kPLoads;
+  // Stores per thread in one epilogue; the first kWB iterations of the next tile add them and
+  // the next tile's perm loads (kXH) to their waits.
+  constexpr int kEpiBlocks = MB <= 4 ? MB : MB / 2;         // 16-row blocks per epilogue pass
+  constexpr int kEpiPasses = MB / kEpiBlocks;
+  constexpr int kRowChunks = (UP ? kPUpCols : kPDnCols) / 8;   // 16-byte pieces of an output row
+  constexpr int kPassStores = (16 * kEpiBlocks * kRowChunks + 64 * kPW - 1) / (64 * kPW);
+  constexpr int kEpiStores = kPassStores * kEpiPasses;
+  constexpr int kXH = kEpiStores + kALoads;
   auto wait_b = [&](int bs, bool head) {
-    constexpr int n = (kWB - 1) * kWOps + kPLoads;
+    constexpr int n = (kWB - 1) * kWOps + kALoads;
     static_assert(kWBLoads == 4 && n + kXH < 64, "four weight registers per stage; vmcnt range");
     if (head)
       asm volatile("s_waitcnt vmcnt(%4)"
@@ -1166,7 +1179,7 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
     dsw16<3 * 1024>(wr_lds, breg[bs][3]);
   };
   auto multiply = [&](int aslot) {
-    const u32x4* la = lA + aslot * kPSlot;
+    const u32x4* la = lA + aslot * kSlot;
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       const int rd = ks ? rd1 : rd0;
@@ -1185,9 +1198,12 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
       // Down: chunks of at most 128 rows (about half the groups at ~128 tokens per expert)
       // skip the last two row blocks, all padding (down 387 -> 369 us at T=4096; the up
       // GEMM showed no gain and keeps one straight-line schedule).
-      static_assert(kPMB == 10, "8 row blocks, then the two that chunks over 128 rows use");
-      blocks(0, 8);
-      if (UP || cur.m > 128) blocks(8, kPMB);
+      if constexpr (MB == 10 && !UP) {
+        blocks(0, 8);
+        if (cur.m > 128) blocks(8, MB);
+      } else {
+        blocks(0, MB);
+      }
     }
   };
   auto barrier_raw = [&]() {
@@ -1206,7 +1222,7 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
     barrier_raw();
   };
 
-  // Epilogue in two passes of five 16-row blocks, row r's 16-byte chunk q at chunk
+  // Epilogue in passes of kEpiBlocks 16-row blocks, row r's 16-byte chunk q at chunk
   // q ^ 2 ((r / 4) % 4); C fragment lane l holds rows 4 (l / 16) + e, column l % 16.
   // Staging: the wave regions (32 KB, free between a tile's last stage and the next tile's
   // first) hold the pass's first kStgRows rows, the A ring slot
@@ -1214,15 +1230,15 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
   // is requested in the next tile's first iteration) the rest.
   auto epilogue = [&](const PTile& t, int free_slot) {
     constexpr int TCB = UP ? 2 * kPUpCols : 2 * kPDnCols;
-    constexpr int BPP = 5;
+    constexpr int BPP = kEpiBlocks;
     constexpr int RPP = 16 * BPP, CPR = TCB / 16;
-    constexpr int NST = (RPP * CPR + 64 * kPW - 1) / (64 * kPW);
+    constexpr int NST = kPassStores;
     constexpr int kStgRows = kPW * kWReg * 16 / TCB;
-    static_assert(kPMB % BPP == 0 && RPP <= kStgRows + kPSlot * 16 / TCB, "a pass fits in the staging");
-    static_assert(NST * 64 * kPW / CPR <= kStgRows + kPSlot * 16 / TCB, "reads past the pass stay in it");
-    static_assert(NST * (kPMB / BPP) == kEpiStores, "stores per thread per epilogue");
+    static_assert(MB % BPP == 0 && RPP <= kStgRows + kSlot * 16 / TCB, "a pass fits in the staging");
+    static_assert(NST * 64 * kPW / CPR <= kStgRows + kSlot * 16 / TCB, "reads past the pass stay in it");
+    static_assert(CPR == kRowChunks && MB == BPP * kEpiPasses, "stores per thread per epilogue");
     char* const stg = reinterpret_cast<char*>(lB);
-    char* const stg2 = reinterpret_cast<char*>(lA + free_slot * kPSlot);
+    char* const stg2 = reinterpret_cast<char*>(lA + free_slot * kSlot);
     auto rowp = [&](int r) { return r < kStgRows ? stg + r * TCB : stg2 + (r - kStgRows) * TCB; };
     const int sw = 2 * (lane >> 4), rl = 4 * (lane >> 4);
     int cb[kPNB];
@@ -1232,7 +1248,7 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
       cb[nb] = ((col >> 3) ^ sw) * 16 + (col & 7) * 2;
     }
 #pragma unroll
-    for (int P = 0; P < kPMB / BPP; ++P) {
+    for (int P = 0; P < MB / BPP; ++P) {
 #pragma unroll
       for (int ii = 0; ii < BPP; ++ii) {
         const int i = P * BPP + ii;
@@ -1322,7 +1338,7 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
     cur = nxt;
     nxt = tile(min(j + 2, ntile - 1));
 #pragma unroll
-    for (int q = 0; q < kPLoads; ++q) a_off_cur[q] = a_off_nxt[q];
+    for (int q = 0; q < kALoads; ++q) a_off_cur[q] = a_off_nxt[q];
     fetch_perm(pv_nxt, nxt);
   }
   wait_vmcnt<0>();
@@ -1430,12 +1446,47 @@ __global__ __launch_bounds__(256) void k_combine(const int32_t* ids32, const int
 // ---------------------------------------------------------------- driver
 int dispatch_launch(const int32_t* ids32, const int64_t* ids64, int T, int k, int E, int shared_rows,
                     int32_t* offsets, int32_t* perm, int32_t* inv, int32_t* tile_start, uint32_t* err,
-                    hipStream_t s, int4* desc) {
+                    hipStream_t s, int4* desc, int bm) {
   if ((long)T * k > kScatterMaxN) return TMOE_ERR_SHAPE;
   hipLaunchKernelGGL(k_dispatch_count, dim3(1), dim3(1024), 0, s, ids32, ids64, T, k, E, shared_rows, offsets,
-                     tile_start, inv, err, desc);
+                     tile_start, inv, err, desc, bm);
   hipLaunchKernelGGL(k_dispatch_scatter, dim3(E), dim3(1024), 0, s, ids32, ids64, T, k, offsets, perm, inv);
   return hipGetLastError() == hipSuccess ? TMOE_OK : TMOE_ERR_HIP;
+}
+
+// The whole-line bf16 kernel's weight stages in registers for a K of nk stages: 4 or 5, whichever
+// divides nk with at least two cycles per tile, 0 if neither.  Where both do: 5 for the up GEMM of
+// 160-row chunks (655 -> 646 us at T=4096), else 4 (with 32- and 64-row chunks, whose smaller
+// accumulators leave room for 8, four stages were faster: T=40 layer 509 us against 520, T=1024
+// 803 against 810, H=2560 E=256 I=1024 k=8).
+static int gemm_w_stages(int nk, bool five_first) {
+  const bool five = nk % 5 == 0 && nk >= 10, four = nk % 4 == 0 && nk >= 8;
+  return five && (five_first || !four) ? 5 : four ? 4 : 0;
+}
+
+template <bool UP, int MB>
+static void gemm_w_launch(const GemmParams& g, unsigned grid, hipStream_t s) {
+  if (gemm_w_stages(g.K / kBK, UP && MB == kBM / 16) == 5)
+    hipLaunchKernelGGL((k_grouped_gemm_w<UP, 5, MB>), dim3(grid), dim3(64 * kPW), 0, s, g);
+  else
+    hipLaunchKernelGGL((k_grouped_gemm_w<UP, 4, MB>), dim3(grid), dim3(64 * kPW), 0, s, g);
+}
+template <bool UP>
+static void gemm_w_launch(const GemmParams& g, int bm, unsigned grid, hipStream_t s) {
+  if (bm == 32) gemm_w_launch<UP, 2>(g, grid, s);
+  else if (bm == 64) gemm_w_launch<UP, 4>(g, grid, s);
+  else gemm_w_launch<UP, kBM / 16>(g, grid, s);
+}
+
+// Rows per M-chunk of the bf16 GEMMs: the fewest (32, 64, 160) that hold a group of the mean
+// size plus three standard deviations of a uniform routing.  A chunk's padding rows cost token-row
+// traffic (L2 -> LDS) and MFMAs next to the weight stream; a group split in two costs a second
+// pass over its weights.  Layer, H=2560 E=256 I=1024 k=8, 160 -> 64 -> 32 rows: T=40 (mean 1.25)
+// 549 -> 521 -> 509 us, T=1024 (mean 32) 842 -> 803 -> 890 us.
+static int chunk_rows(int T, int k, int E) {
+  const float mean = (float)T * (float)k / (float)E;
+  const float want = mean + 3.0f * sqrtf(mean);
+  return want <= 32.0f ? 32 : want <= 64.0f ? 64 : kBM;
 }
 
 int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t* ids64, const float* wf,
@@ -1457,11 +1508,28 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
   uint16_t* ch = ws_ptr<uint16_t>(ws, L.ch);
   uint16_t* sh = ws_ptr<uint16_t>(ws, L.sh);
   int4* desc = ws_ptr<int4>(ws, L.desc);
+  const int n_groups = has_sh ? E + 1 : E;
+  // A rows are addressed with 32-bit byte offsets by the persistent kernels.
+  const bool ofs32 = (size_t)T * H * 2 < ((size_t)1 << 32) && ((size_t)T * k + T) * I * 2 < ((size_t)1 << 32);
+  static const bool frag = [] {
+    const char* e = getenv("TMOE_PREFILL_GEMM");
+    return e && !strcmp(e, "frag");
+  }();
+  // Whole-line kernel: 128 activation columns (up) or 256 output columns (down) per tile.
+  const bool line = I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32 && gemm_w_stages(H / kBK, true) &&
+                    gemm_w_stages(I / kBK, true);
+  int bm = q4 || frag || !line ? kBM : chunk_rows(T, k, E);
+  if (bm != kBM) {
+    // More chunks than the descriptor region holds (T k / 64): the router logits' region, read
+    // for the last time by the top-k launch, takes them.
+    const size_t chunks = (size_t)T * k / bm + (size_t)n_groups + T / bm + 2;
+    if (16 * chunks <= sizeof(float) * (size_t)T * (E + 1)) desc = ws_ptr<int4>(ws, L.logits);
+    else bm = kBM;
+  }
   if (int st = dispatch_launch(ids32, ids64, T, k, E, has_sh ? T : 0, offsets, perm, inv, tile_start, err, s,
-                               desc))
+                               desc, bm))
     return st;
 
-  const int n_groups = has_sh ? E + 1 : E;
   const long mbound = (long)T * k / kBM + (long)(E < T * k ? E : T * k) + (has_sh ? (T + kBM - 1) / kBM : 0) + 1;
   const long mshared = (T + kBM - 1) / kBM;
 
@@ -1472,21 +1540,15 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
   // A rows with 32-bit byte offsets; other shapes take the register-staged kernel (64 and
   // 128 columns).
   const int kcyc = kBK * kPR;
-  const bool persistent = H % kcyc == 0 && I % kcyc == 0 && I % kPUpCols == 0 && H % kPDnCols == 0 &&
-                          (size_t)T * H * 2 < ((size_t)1 << 32) && ((size_t)T * k + T) * I * 2 < ((size_t)1 << 32);
-  const int up_cols = persistent ? kPUpCols : 64, dn_cols = persistent ? kPDnCols : 128;
+  const bool persistent = H % kcyc == 0 && I % kcyc == 0 && I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32;
   static int n_cu[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return TMOE_ERR_HIP;
   if (!n_cu[dev] && hipDeviceGetAttribute(&n_cu[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return TMOE_ERR_HIP;
   const unsigned pgrid = (unsigned)(n_cu[dev] >= 8 ? n_cu[dev] / 8 * 8 : 8);
-  // bf16 groups of the persistent shapes run on the whole-line kernel; TMOE_PREFILL_GEMM=frag
-  // selects the fragment-load kernel for them (int4 groups always use it).
-  static const bool frag = [] {
-    const char* e = getenv("TMOE_PREFILL_GEMM");
-    return e && !strcmp(e, "frag");
-  }();
+  // bf16 groups run on the whole-line kernel where it takes the shape; TMOE_PREFILL_GEMM=frag
+  // selects the fragment-load kernel (int4 groups always use it).
   auto gemm = [&](GemmParams g, int lo, int hi, bool routed_q4, long mchunks) {
     g.group_lo = lo;
     g.group_hi = hi;
@@ -1494,8 +1556,8 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
     // after requesting them, so an up GEMM it would run over K < 2 kPR stages (H = 512) runs
     // on the register-staged kernel instead, with its narrower tiles.
     const bool frag_kernel = routed_q4 || frag;
-    const bool staged = !persistent || (frag_kernel && g.up && g.K < 2 * kcyc);
-    if (persistent && staged) g.n_ntiles = g.up ? I / 64 : H / 128;
+    const bool staged = frag_kernel ? !persistent || (g.up && g.K < 2 * kcyc) : !line;
+    g.n_ntiles = g.up ? I / (staged ? 64 : kPUpCols) : H / (staged ? 128 : kPDnCols);
     const long grid = (mchunks * g.n_ntiles + 7) / 8 * 8;
     if (staged) {
       if (routed_q4 && qr)
@@ -1510,22 +1572,20 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
       hipLaunchKernelGGL((k_grouped_gemm_p<true>), dim3(pgrid), dim3(64 * kPW), 0, s, g);
     } else if (frag) {
       hipLaunchKernelGGL((k_grouped_gemm_p<false>), dim3(pgrid), dim3(64 * kPW), 0, s, g);
-    } else if (g.up && g.K % (5 * kBK) == 0) {
-      hipLaunchKernelGGL((k_grouped_gemm_w<true, 5>), dim3(pgrid), dim3(64 * kPW), 0, s, g);
     } else if (g.up) {
-      hipLaunchKernelGGL((k_grouped_gemm_w<true, 4>), dim3(pgrid), dim3(64 * kPW), 0, s, g);
+      gemm_w_launch<true>(g, bm, pgrid, s);
     } else {
-      hipLaunchKernelGGL((k_grouped_gemm_w<false, 4>), dim3(pgrid), dim3(64 * kPW), 0, s, g);
+      gemm_w_launch<false>(g, bm, pgrid, s);
     }
   };
   GemmParams up{};
   up.a = x; up.K = H; up.gather = 1; up.offsets = offsets; up.perm = perm; up.tile_start = tile_start;
-  up.T = T; up.E = E; up.k = k; up.n_groups = n_groups; up.n_ntiles = I / up_cols; up.up = 1; up.N = I; up.I = I;
+  up.T = T; up.E = E; up.k = k; up.n_groups = n_groups; up.up = 1; up.N = I; up.I = I;
   up.table = table; up.shw0 = sh_gate; up.shw1 = sh_up; up.shared_row0 = T * k; up.out = act;
   up.desc = desc;
   up.sink = reinterpret_cast<uint16_t*>(tile_start + ((E + 5) & ~3));   // past tile_start's E + 2 words
   GemmParams dn = up;
-  dn.a = act; dn.K = I; dn.gather = 0; dn.n_ntiles = H / dn_cols; dn.up = 0; dn.N = H;
+  dn.a = act; dn.K = I; dn.gather = 0; dn.up = 0; dn.N = H;
   dn.shw0 = sh_down; dn.shw1 = nullptr; dn.out = ch; dn.out_sh = sh;
   if (q4) {
     gemm(up, 0, E, true, mbound);
@@ -1572,5 +1632,5 @@ extern "C" int tmoe_dispatch(const int64_t* ids, int T, int k, int E, int32_t* o
   const Ws L = ws_layout(T, 8, E, 8, k, 0);
   if (ws_bytes < L.scratch + sizeof(int32_t) * (size_t)(E + 64)) return TMOE_ERR_WORKSPACE;
   return dispatch_launch(nullptr, ids, T, k, E, 0, offsets, perm, inv, ws_ptr<int32_t>(workspace, L.scratch),
-                         ws_ptr<uint32_t>(workspace, L.status) + kStatusError, (hipStream_t)stream, nullptr);
+                         ws_ptr<uint32_t>(workspace, L.status) + kStatusError, (hipStream_t)stream, nullptr, kBM);
 }
