@@ -45,11 +45,12 @@ __device__ __forceinline__ bool ids_aligned(const int32_t* ids32, const int64_t*
 
 // ---------------------------------------------------------------- dispatch
 // One block of 1024 threads: per-expert counts, offsets, M-chunk schedule, inv := -1, and
-// (desc non-null) one descriptor per M-chunk of bm rows: {group, rows, first row in group order, 0}.
+// (desc non-null) one descriptor per M-chunk (bm rows, the shared
+// group's bms): {group, rows, first row in group order, 0}.
 __global__ __launch_bounds__(1024) void k_dispatch_count(const int32_t* ids32, const int64_t* ids64, int T, int k,
                                                          int E, int shared_rows, int32_t* offsets,
                                                          int32_t* tile_start, int32_t* inv, uint32_t* err,
-                                                         int4* desc, int bm) {
+                                                         int4* desc, int bm, int bms) {
   __shared__ int cnt[1024];
   const int tid = threadIdx.x;
   for (int e = tid; e < 1024; e += 1024) cnt[e] = 0;
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(1024) void k_dispatch_count(const int32_t* ids32, c
   __syncthreads();
   // Inclusive Hillis-Steele scans of counts and M-chunks (groups 0..E-1, then the shared group).
   const int c = tid < E ? cnt[tid] : 0;
-  int ch = tid < E ? (c + bm - 1) / bm : (tid == E ? (shared_rows + bm - 1) / bm : 0);
+  int ch = tid < E ? (c + bm - 1) / bm : (tid == E ? (shared_rows + bms - 1) / bms : 0);
   __shared__ int sc[1024], sk[1025];
   sc[tid] = c;
   sk[tid] = ch;
@@ -104,7 +105,7 @@ __global__ __launch_bounds__(1024) void k_dispatch_count(const int32_t* ids32, c
   if (tid == 0) { offsets[0] = 0; tile_start[0] = 0; }
   if (tid <= E) tile_start[tid + 1] = sk[tid];
   if (!desc) return;
-  // M-chunk mt of group g (sk[g - 1] <= mt < sk[g]): rows r0 = (mt - sk[g - 1]) bm onwards.
+  // M-chunk mt of group g (sk[g - 1] <= mt < sk[g]): rows r0 = (mt - sk[g - 1]) gm onwards.
   const int n_groups = shared_rows > 0 ? E + 1 : E;
   const int n_chunks = sk[n_groups - 1];
   for (int mt = tid; mt < n_chunks; mt += 1024) {
@@ -114,10 +115,11 @@ __global__ __launch_bounds__(1024) void k_dispatch_count(const int32_t* ids32, c
       if (sk[mid] > mt) hi = mid; else lo = mid + 1;
     }
     const int g = lo;
-    const int r0 = (mt - (g ? sk[g - 1] : 0)) * bm;
+    const int gm = g < E ? bm : bms;
+    const int r0 = (mt - (g ? sk[g - 1] : 0)) * gm;
     const int rows = g < E ? cnt[g] : shared_rows;
     const int first = g < E ? (g ? sc[g - 1] : 0) : 0;
-    desc[mt] = int4{g, min(bm, rows - r0), first + r0, 0};
+    desc[mt] = int4{g, min(gm, rows - r0), first + r0, 0};
   }
 }
 
@@ -203,6 +205,7 @@ struct GemmParams {
   uint16_t* out;             // up: act; down: ch [T*k, H], each expert output unscaled
   uint16_t* out_sh;          // down: sh [T, H], the shared expert's output before its gate
   const int4* desc;          // persistent kernel: M-chunk descriptors {group, rows, first row, 0}
+  int sh_blocks;             // int4 small-group launch: blocks that run the shared group's (bf16) tiles
   uint16_t* sink;            // 16 bytes nobody reads: whole-line kernel stores of rows past a tile
 };
 
@@ -215,18 +218,26 @@ __device__ __forceinline__ bf16x8_t as_bf16x8(u32x4 v) { return __builtin_bit_ca
 // bf16 (v_cvt_pk_bf16_f32, two values per instruction) reproduces the dequantised matrix
 // bit for bit (finite scales).
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+// Two nibbles (bytes 2 W and 2 W + 1 of v, each 0..15) as fp32 in one conversion: a byte 0..15 read
+// as fp8 e4m3 is exactly n 2^-9 (0..7 its denormals, 8..15 its first binade), scaled here by 2^9.
+// v_cvt_f32_ubyte takes as long for one (both ~6 cycles a wave, fp32 FMA ~3.4, in a probe of four
+// waves per SIMD), so the conversions are half as many: 11 of the slower instructions per 8 weights
+// against 15 (20 as the compiler wrote the byte extracts).
+template <bool W>
+__device__ __forceinline__ f32x2 nibbles_f32(uint32_t v) {
+  return __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)v, 512.0f, W);
+}
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+  return __builtin_bit_cast(uint32_t, bf16x2_t{(__bf16)a, (__bf16)b});
+}
 __device__ __forceinline__ u32x4 dequant_frag(uint32_t w, float s) {
-  const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+  const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;   // even k, odd k
   const float m8 = -8.0f * s;
-  uint32_t d[4];
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const float e = fmaf((float)((lo >> (8 * b)) & 0xFFu), s, m8);
-    const float o = fmaf((float)((hi >> (8 * b)) & 0xFFu), s, m8);
-    const bf16x2_t v = {(__bf16)e, (__bf16)o};   // (even k low, odd k high)
-    d[b] = __builtin_bit_cast(uint32_t, v);
-  }
-  return u32x4{d[0], d[1], d[2], d[3]};
+  const f32x2 l0 = nibbles_f32<false>(lo), l1 = nibbles_f32<true>(lo);
+  const f32x2 h0 = nibbles_f32<false>(hi), h1 = nibbles_f32<true>(hi);
+  return u32x4{bf16_pair(fmaf(l0.x, s, m8), fmaf(h0.x, s, m8)), bf16_pair(fmaf(l0.y, s, m8), fmaf(h0.y, s, m8)),
+               bf16_pair(fmaf(l1.x, s, m8), fmaf(h1.x, s, m8)), bf16_pair(fmaf(l1.y, s, m8), fmaf(h1.y, s, m8))};
 }
 // A scale's 16 bits as fp32: bf16 (group scales) or fp16 (QR, per-row scales).
 template <bool QR>
@@ -552,6 +563,18 @@ __device__ __forceinline__ uint32_t gld2(const void* sbase, uint32_t voff) {
   asm volatile("global_load_ushort %0, %1, %2" : "=v"(v) : "v"(voff), "s"(sbase));
   return v;
 }
+// The same into a register that keeps its place (tied to its old value), for loads that several
+// paths of a loop leave in flight: with a fresh result the compiler may join the paths by copies,
+// which would read the register before the load has landed.
+__device__ __forceinline__ void gld16_into(u32x4& v, const void* sbase, uint32_t voff) {
+  asm volatile("global_load_dwordx4 %0, %1, %2" : "+v"(v) : "v"(voff), "s"(sbase));
+}
+__device__ __forceinline__ void gld4_into(uint32_t& v, const void* sbase, uint32_t voff) {
+  asm volatile("global_load_dword %0, %1, %2" : "+v"(v) : "v"(voff), "s"(sbase));
+}
+__device__ __forceinline__ void gld2_into(uint32_t& v, const void* sbase, uint32_t voff) {
+  asm volatile("global_load_ushort %0, %1, %2" : "+v"(v) : "v"(voff), "s"(sbase));
+}
 // 16 bytes per lane from global memory straight into LDS at lds + 16 lane (M0 = lds).
 // Nothing else in the kernel uses M0.
 __device__ __forceinline__ void gdma16(const void* sbase, uint32_t voff, const void* lds) {
@@ -807,6 +830,7 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_p(GemmParams p) {
     for (int nb = 0; nb < kPNB; ++nb) bc[nb] = as_bf16x8(cur_b[nb]);
     uint32_t lo[kPNB], hi[kPNB];
     float sc[kPNB], m8[kPNB];
+    f32x2 le, ho;
     // Chunks of at most 128 rows skip the MFMAs of the last two row blocks (all padding).
     static_assert(kPMB == 10, "8 row blocks, then the two that chunks over 128 rows use");
     const bool full = cur.m > 128;
@@ -835,10 +859,10 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_p(GemmParams p) {
         }
       } else if (i <= 4 * kPNB) {
         const int w = i - 1, nb = w / 4, b = w % 4;
-        const float e = fmaf((float)((lo[nb] >> (8 * b)) & 0xFFu), sc[nb], m8[nb]);
-        const float o = fmaf((float)((hi[nb] >> (8 * b)) & 0xFFu), sc[nb], m8[nb]);
-        const bf16x2_t v = {(__bf16)e, (__bf16)o};   // (even k low, odd k high)
-        const uint32_t d = __builtin_bit_cast(uint32_t, v);
+        // Words 2 i and 2 i + 1 share two conversions; (even k low, odd k high).
+        if (b == 0) { le = nibbles_f32<false>(lo[nb]); ho = nibbles_f32<false>(hi[nb]); }
+        if (b == 2) { le = nibbles_f32<true>(lo[nb]); ho = nibbles_f32<true>(hi[nb]); }
+        const uint32_t d = bf16_pair(fmaf(le[b & 1], sc[nb], m8[nb]), fmaf(ho[b & 1], sc[nb], m8[nb]));
         if (b == 0) nxt_b[nb].x = d;
         else if (b == 1) nxt_b[nb].y = d;
         else if (b == 2) nxt_b[nb].z = d;
@@ -1022,16 +1046,20 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_p(GemmParams p) {
 constexpr int kWBLoads = 2 * kPNB;            // weight loads per wave per stage (8 rows each)
 constexpr int kWReg = 16 * kPNB * 8;          // u32x4 per wave region (32 rows x 128 B)
 
+template <int WB, int MB>
+constexpr int kWLdsA = (WB + 1) * MB * 16 * 8;   // u32x4 of the A ring
+constexpr int kWLdsB = kPW * kWReg;              // and of the wave regions
+
+// Block bid of nblk walking groups [p.group_lo, p.group_hi).
 template <bool UP, int WB, int MB>
-__global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
+__device__ __forceinline__ void gemm_w_body(const GemmParams& p, int bid, int nblk, u32x4* const lA, u32x4* const lB) {
   constexpr int kWB = WB, kWA = WB, kWAS = WB + 1;
   constexpr int kSlot = MB * 16 * 8;             // u32x4 per A slot (16 MB rows x 128 B)
   constexpr int kALoads = (2 * MB + kPW - 1) / kPW;   // A loads per wave per stage
   constexpr int kWOps = kALoads + kWBLoads;      // vector memory operations per stage
   static_assert(kWBLoads + (kWA - 1) * kWOps < 64 && (kWB - 1) * kWOps + kALoads < 64, "vmcnt range");
   static_assert((kWAS * kSlot + kPW * kWReg) * 16 <= 160 * 1024, "LDS");
-  __shared__ u32x4 lA[kWAS * kSlot];
-  __shared__ u32x4 lB[kPW * kWReg];
+  static_assert(kWLdsA<WB, MB> == kWAS * kSlot, "A ring");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int K = p.K;
@@ -1044,8 +1072,8 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
   const int c_lo = sload1(p.tile_start + p.group_lo);
   const int c_hi = sload1(p.tile_start + p.group_hi);
   const int total = (c_hi - c_lo) * p.n_ntiles;
-  const int nbx = (int)gridDim.x >> 3;
-  const int xcd = (int)blockIdx.x & 7, qb = (int)blockIdx.x >> 3;
+  const int nbx = nblk >> 3;
+  const int xcd = bid & 7, qb = bid >> 3;
   const int per_xcd = (total + 7) / 8;
   const int f0 = xcd * per_xcd + qb;
   const int f_end = min(total, (xcd + 1) * per_xcd);
@@ -1344,6 +1372,338 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
   wait_vmcnt<0>();
 }
 
+template <bool UP, int WB, int MB>
+__global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
+  __shared__ u32x4 lA[kWLdsA<WB, MB>];
+  __shared__ u32x4 lB[kWLdsB];
+  gemm_w_body<UP, WB, MB>(p, (int)blockIdx.x, (int)gridDim.x, lA, lB);
+}
+
+// ---------------------------------------------------------------- grouped GEMM, int4, small groups
+// Int4 groups of up to 64 rows (k_grouped_gemm_p's 160-row tiles would read and multiply mostly
+// padding).  Tiles as in the kernels above: 16 MB rows of one group x 8 waves x 32 weight rows.
+//   K stage: 128, one scale group.  A lane takes 16 bytes of its weight row per stage and 16-row
+//   block in one load (lane group g = lane / 16: k 32 g .. 32 g + 31; its word s is the B fragment of
+//   k step s), so a load reads 16 rows x 64 bytes; the A fragment of k step s is 16-byte chunk
+//   4 g + s of the stage's 256-byte rows (the same permutation of k for both operands).
+//   A: global -> LDS, 4 rows x 256 bytes per load, row r's chunk c at chunk c ^ (r % 16); a ring of
+//   kQB + 1 slots requested kQB stages ahead, as the weights (in registers).
+// What bounds it is the dequantisation (~23 VALU instructions per 8 weights and lane) beside the
+// weight stream, so two blocks share a CU (128 registers a wave): one block's waits and epilogues
+// overlap the other's arithmetic.
+// The stages of a block's tiles form one stream: stage sc of a tile requests stage sc + kQB, the next
+// tile's first ones past the tile's end.  A tile may have any number of stages >= kQB: a tile's row
+// indices are fetched two tiles ahead, at least kQB stage waits before they are used.
+constexpr int kQK = 128;
+constexpr int kQB = 4;
+constexpr int kQShared = 32;   // rows per chunk of the shared group beside them
+
+struct QTile {
+  int arow0, m;             // A row of the first row (up: its position in perm); valid rows
+  const uint8_t* q[kPNB];   // this wave's packed weight rows
+  const uint16_t* sc[kPNB]; // and their scales
+  uint16_t* o;              // first output row, this tile's first column
+};
+
+template <int MB>
+constexpr int kQLds = (kQB + 1) * (MB < 2 ? 2 : MB) * 16 * 16;   // u32x4 of the A ring
+
+template <bool UP, bool QR, int MB>
+__device__ __forceinline__ void gemm_q_body(const GemmParams& p, int bid, int nblk, u32x4* const lA) {
+  constexpr int kSlot = (MB < 2 ? 2 : MB) * 16 * 16;       // u32x4 per A slot (16 MB rows x 256 B, at least 8 KB)
+  constexpr int kAS = kQB + 1;
+  constexpr int kALoads = (4 * MB + kPW - 1) / kPW;        // A loads per wave per stage
+  constexpr int kBLoads = QR ? kPNB : 2 * kPNB;            // packed rows, and the group scales
+  constexpr int kOps = kALoads + kBLoads;
+  static_assert(4 * MB % kPW == 0 || 4 * MB == kPW / 2, "A loads: each part once, or by two waves");
+  static_assert(kQLds<MB> == kAS * kSlot, "A ring");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int K = p.K, nk = K / kQK;
+
+  const int c_lo = sload1(p.tile_start + p.group_lo);
+  const int c_hi = sload1(p.tile_start + p.group_hi);
+  const int total = (c_hi - c_lo) * p.n_ntiles;
+  const int nbx = nblk >> 3;
+  const int xcd = bid & 7, qb = bid >> 3;
+  const int per_xcd = (total + 7) / 8;
+  const int f0 = xcd * per_xcd + qb;
+  const int f_end = min(total, (xcd + 1) * per_xcd);
+  if (f0 >= f_end) return;
+  const int ntile = (f_end - f0 + nbx - 1) / nbx;
+
+  auto chunk = [&](int j) {        // tile j's M-chunk descriptor (the last tile's past the end)
+    return sload4(p.desc + c_lo + (f0 + min(j, ntile - 1) * nbx) / p.n_ntiles);
+  };
+  auto tile = [&](int j) {
+    j = min(j, ntile - 1);
+    const int nt = (f0 + j * nbx) % p.n_ntiles;
+    const i32x4 d = chunk(j);
+    QTile t;
+    t.m = d.y;
+    t.arow0 = d.z;
+    const int c0 = UP ? nt * kPUpCols + wid * 16 : nt * kPDnCols + wid * 32;
+    t.o = p.out + (size_t)d.z * p.N + nt * (UP ? kPUpCols : kPDnCols);
+    const uint64_t* te = p.table + 4 * d.x + (UP ? 0 : 2);
+    const uint8_t* pk = reinterpret_cast<const uint8_t*>(sload_ptr(te));
+    const uint16_t* sc = reinterpret_cast<const uint16_t*>(sload_ptr(te + 1));
+#pragma unroll
+    for (int nb = 0; nb < kPNB; ++nb) {
+      const int wr = UP ? (nb ? p.I : 0) + c0 : c0 + 16 * nb;
+      t.q[nb] = pk + (size_t)wr * (K / 2);
+      t.sc[nb] = sc + (size_t)wr * (QR ? 1 : K / kQK);
+    }
+    return t;
+  };
+
+  // Lane constants.  A load j of this wave: rows 4 x .. 4 x + 3, x = wid + 8 j (MB = 1: waves 4-7
+  // repeat parts 0-3, the same bytes to the same place).
+  const int lrow = lane & 15, lg = lane >> 4;
+  int a_part[kALoads], a_row[kALoads];
+  uint32_t a_col[kALoads];
+#pragma unroll
+  for (int j = 0; j < kALoads; ++j) {
+    a_part[j] = MB == 1 ? (wid & 3) : wid + kPW * j;
+    a_row[j] = 4 * a_part[j] + lg;
+    a_col[j] = 16u * (uint32_t)(lrow ^ (a_row[j] & 15));
+  }
+  int a_rd[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) a_rd[s] = lrow * 16 + ((4 * lg + s) ^ lrow);
+  const uint32_t q_off = (uint32_t)(lrow * (K / 2) + 16 * lg);
+  const uint32_t s_off = (uint32_t)(lrow * (QR ? 1 : K / kQK) * 2);
+
+  f32x4 acc[MB][kPNB];
+  auto zero_acc = [&]() {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int nb = 0; nb < kPNB; ++nb) acc[i][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  zero_acc();
+
+  u32x4 bq[kQB][kPNB];
+  uint32_t sreg[kQB][kPNB], srow[kPNB] = {};   // group scales in flight; QR: the next tile's row scales
+  float rs[kPNB] = {};                          // QR: this tile's row scales
+#pragma unroll
+  for (int v = 0; v < kQB; ++v)
+#pragma unroll
+    for (int nb = 0; nb < kPNB; ++nb) {
+      bq[v][nb] = u32x4{0u, 0u, 0u, 0u};
+      sreg[v][nb] = 0u;
+    }
+  uint32_t a_off_cur[kALoads], a_off_nxt[kALoads], pv[kALoads] = {};
+  auto fetch_perm = [&](int arow0, int m) {
+    if constexpr (UP) {
+      const int32_t* pp = p.perm + arow0;
+#pragma unroll
+      for (int j = 0; j < kALoads; ++j) gld4_into(pv[j], pp, (uint32_t)(min(a_row[j], m - 1) * 4));
+    }
+  };
+  auto a_offsets = [&](uint32_t* o, const QTile& t) {
+#pragma unroll
+    for (int j = 0; j < kALoads; ++j) {
+      int row = t.arow0 + min(a_row[j], t.m - 1);
+      if constexpr (UP) row = (int)pv[j] / p.k;
+      o[j] = (uint32_t)row * (uint32_t)(K * 2) + a_col[j];
+    }
+  };
+  auto fetch_srow = [&](const QTile& t) {
+    if constexpr (QR) {
+#pragma unroll
+      for (int nb = 0; nb < kPNB; ++nb) gld2_into(srow[nb], t.sc[nb], s_off);
+    }
+  };
+  // Waits for everything but the last kBLoads + (kQB - 1) kOps operations (a stage end's count), the
+  // row indices and row scales passed through it.
+  auto wait_fetched = [&]() {
+    constexpr int n = kBLoads + (kQB - 1) * kOps;
+    if constexpr (UP && kALoads == 2) asm volatile("s_waitcnt vmcnt(%2)" : "+v"(pv[0]), "+v"(pv[kALoads - 1]) : "n"(n));
+    else if constexpr (UP) asm volatile("s_waitcnt vmcnt(%1)" : "+v"(pv[0]) : "n"(n));
+    if constexpr (QR) asm volatile("s_waitcnt vmcnt(%2)" : "+v"(srow[0]), "+v"(srow[1]) : "n"(n));
+  };
+  auto take_srow = [&]() {
+    if constexpr (QR) {
+#pragma unroll
+      for (int nb = 0; nb < kPNB; ++nb) rs[nb] = scale_f32<true>((uint16_t)srow[nb]);
+    }
+  };
+  QTile cur, nxt;
+  auto dma_a = [&](int slot, bool nx, int st) {
+    const char* ta = reinterpret_cast<const char*>(p.a) + (size_t)st * kQK * 2;
+#pragma unroll
+    for (int j = 0; j < kALoads; ++j)
+      gdma16(ta, nx ? a_off_nxt[j] : a_off_cur[j], lA + slot * kSlot + a_part[j] * 64);
+  };
+  auto load_b = [&](int bs, bool nx, int st) {
+#pragma unroll
+    for (int nb = 0; nb < kPNB; ++nb) {
+      gld16_into(bq[bs][nb], (nx ? nxt.q[nb] : cur.q[nb]) + (size_t)st * (kQK / 2), q_off);
+      if constexpr (!QR) gld2_into(sreg[bs][nb], (nx ? nxt.sc[nb] : cur.sc[nb]) + st, s_off);
+    }
+  };
+  auto barrier_raw = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // Weight stage bs was requested kQB stages ago: the kQB - 1 later stages' operations and this
+  // stage's A loads may be outstanding (stricter right after an epilogue's stores).  The registers
+  // pass through the asm, so nothing reads them before the wait.
+  auto multiply = [&](int bs, int slot) {
+    constexpr int n = (kQB - 1) * kOps + kALoads;
+    static_assert(n < 64, "vmcnt range");
+    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(bq[bs][0]), "+v"(bq[bs][1]) : "n"(n));
+    float sc[kPNB];
+#pragma unroll
+    for (int nb = 0; nb < kPNB; ++nb) {
+      if constexpr (!QR) asm volatile("" : "+v"(sreg[bs][nb]));
+      sc[nb] = QR ? rs[nb] : scale_f32<false>((uint16_t)sreg[bs][nb]);
+    }
+    const u32x4* la = lA + slot * kSlot;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      bf16x8_t b[kPNB];
+#pragma unroll
+      for (int nb = 0; nb < kPNB; ++nb) b[nb] = as_bf16x8(dequant_frag(bq[bs][nb][s], sc[nb]));
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const bf16x8_t a = as_bf16x8(la[i * 256 + a_rd[s]]);
+#pragma unroll
+        for (int nb = 0; nb < kPNB; ++nb)
+          acc[i][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[nb], acc[i][nb], 0, 0, 0);
+      }
+    }
+  };
+  // This wave's part of the next A stage landed (requested kQB - 1 stages ago, then that stage's
+  // weight loads and kQB - 1 whole stages), then a raw barrier: every wave's part visible, every
+  // wave done reading the slot refilled next.
+  auto stage_end = [&]() {
+    constexpr int n = kBLoads + (kQB - 1) * kOps;
+    static_assert(n < 64, "vmcnt range");
+    wait_vmcnt<n>();
+    barrier_raw();
+  };
+  // Epilogue through the A slot that the tile's last stage used (no load targets it until the next
+  // stage): row r's 16-byte chunk q at chunk q ^ 2 ((r / 4) % 4); C fragment lane l holds rows
+  // 4 (l / 16) + e, column l % 16 of each block.
+  auto epilogue = [&](int slot) {
+    constexpr int TCB = UP ? 2 * kPUpCols : 2 * kPDnCols, CPR = TCB / 16;
+    constexpr int BPP = UP || MB == 1 ? MB : MB / 2, RPP = 16 * BPP;
+    static_assert(RPP * TCB <= kSlot * 16 && MB % BPP == 0, "a pass fits in one ring slot");
+    char* stg = reinterpret_cast<char*>(lA + slot * kSlot);
+    const int sw = 2 * lg, rl = 4 * lg;
+#pragma unroll
+    for (int P = 0; P < MB / BPP; ++P) {
+#pragma unroll
+      for (int ii = 0; ii < BPP; ++ii) {
+        const int i = P * BPP + ii;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          char* rowp = stg + (ii * 16 + rl + e) * TCB;
+          if constexpr (UP) {
+            const int col = wid * 16 + lrow;
+            *reinterpret_cast<uint16_t*>(rowp + ((col >> 3) ^ sw) * 16 + (col & 7) * 2) =
+                swiglu_bits_hw(acc[i][0][e], acc[i][1][e]);
+          } else {
+            const uint32_t w = bf16x2_bits_hw(acc[i][0][e], acc[i][1][e]);
+            const int c0 = wid * 32 + lrow, c1 = c0 + 16;
+            *reinterpret_cast<uint16_t*>(rowp + ((c0 >> 3) ^ sw) * 16 + (c0 & 7) * 2) = (uint16_t)w;
+            *reinterpret_cast<uint16_t*>(rowp + ((c1 >> 3) ^ sw) * 16 + (c1 & 7) * 2) = (uint16_t)(w >> 16);
+          }
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      barrier_raw();
+      for (int x = tid; x < RPP * CPR; x += 64 * kPW) {
+        const int rr = x / CPR, qc = x - rr * CPR, row = P * RPP + rr;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(stg + rr * TCB + ((qc ^ (2 * ((rr >> 2) & 3))) * 16));
+        if (row < cur.m) *reinterpret_cast<u32x4*>(cur.o + (size_t)row * p.N + qc * 8) = v;
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      barrier_raw();
+    }
+  };
+
+  cur = tile(0);
+  nxt = tile(1);
+  fetch_perm(cur.arow0, cur.m);
+  fetch_srow(cur);
+  wait_vmcnt<0>();
+  wait_fetched();
+  a_offsets(a_off_cur, cur);
+  take_srow();
+  fetch_perm(nxt.arow0, nxt.m);
+  fetch_srow(nxt);
+  wait_vmcnt<0>();
+  wait_fetched();
+  a_offsets(a_off_nxt, nxt);
+  {
+    const i32x4 d = chunk(2);
+    fetch_perm(d.z, d.y);
+  }
+#pragma unroll
+  for (int v = 0; v < kQB; ++v) {
+    dma_a(v, false, v);
+    load_b(v, false, v);
+  }
+  stage_end();
+  // Whole cycles of kQB stages: past the last tile's end, stages of repeated data (fewer than kQB
+  // <= nk, so no further epilogue).
+  const int cycles = (ntile * nk + kQB - 1) / kQB;
+  int slot = 0, sc = 0, j = 0;
+  for (int c = 0; c < cycles; ++c) {
+#pragma unroll
+    for (int u = 0; u < kQB; ++u) {
+      const int si = sc + kQB;
+      const bool nx = si >= nk;
+      const int st = nx ? si - nk : si;
+      dma_a(slot == 0 ? kAS - 1 : slot - 1, nx, st);
+      multiply(u, slot);
+      load_b(u, nx, st);
+      stage_end();
+      if (__builtin_expect(++sc == nk, 0)) {
+        epilogue(slot);
+        zero_acc();
+        ++j;
+        cur = nxt;
+        nxt = tile(j + 1);
+        // The next tile's row indices and this one's row scales were requested at the previous
+        // tile's start, at least kQB stages ago.
+        wait_fetched();
+#pragma unroll
+        for (int q = 0; q < kALoads; ++q) a_off_cur[q] = a_off_nxt[q];
+        a_offsets(a_off_nxt, nxt);
+        take_srow();
+        const i32x4 d = chunk(j + 2);
+        fetch_perm(d.z, d.y);
+        fetch_srow(nxt);
+        sc = 0;
+      }
+      slot = slot == kAS - 1 ? 0 : slot + 1;
+    }
+  }
+  wait_vmcnt<0>();   // the unused stages landed before the block's LDS is released
+}
+
+// The routed int4 groups, and beside them the shared expert's bf16 tiles on the first p.sh_blocks
+// blocks (a multiple of 8): as launches of their own these took 46 + 24 us at T = 12, a few blocks
+// streaming 15.7 MB while the rest of the chip idled.
+template <bool UP, bool QR, int MB>
+__global__ __launch_bounds__(64 * kPW, 4) void k_grouped_gemm_q(GemmParams p) {
+  constexpr int kShLds = kWLdsA<4, kQShared / 16> + kWLdsB;
+  __shared__ u32x4 lds[MB >= 4 || kQLds<MB> > kShLds ? kQLds<MB> : kShLds];
+  if (MB < 4 && (int)blockIdx.x < p.sh_blocks) {   // 64-row chunks: never beside the shared group
+    if constexpr (MB < 4) {
+      p.group_lo = p.E;
+      p.group_hi = p.E + 1;
+      gemm_w_body<UP, 4, kQShared / 16>(p, (int)blockIdx.x, p.sh_blocks, lds, lds + kWLdsA<4, kQShared / 16>);
+    }
+  } else {
+    gemm_q_body<UP, QR, MB>(p, (int)blockIdx.x - p.sh_blocks, (int)gridDim.x - p.sh_blocks, lds);
+  }
+}
+
 // ---------------------------------------------------------------- combine
 // One wave per token; lane owns 8 columns per 512-column chunk.  The GEMMs leave each
 // assignment's expert output and the shared expert's output unscaled (bf16 of the fp32
@@ -1446,10 +1806,10 @@ __global__ __launch_bounds__(256) void k_combine(const int32_t* ids32, const int
 // ---------------------------------------------------------------- driver
 int dispatch_launch(const int32_t* ids32, const int64_t* ids64, int T, int k, int E, int shared_rows,
                     int32_t* offsets, int32_t* perm, int32_t* inv, int32_t* tile_start, uint32_t* err,
-                    hipStream_t s, int4* desc, int bm) {
+                    hipStream_t s, int4* desc, int bm, int bms) {
   if ((long)T * k > kScatterMaxN) return TMOE_ERR_SHAPE;
   hipLaunchKernelGGL(k_dispatch_count, dim3(1), dim3(1024), 0, s, ids32, ids64, T, k, E, shared_rows, offsets,
-                     tile_start, inv, err, desc, bm);
+                     tile_start, inv, err, desc, bm, bms);
   hipLaunchKernelGGL(k_dispatch_scatter, dim3(E), dim3(1024), 0, s, ids32, ids64, T, k, offsets, perm, inv);
   return hipGetLastError() == hipSuccess ? TMOE_OK : TMOE_ERR_HIP;
 }
@@ -1478,15 +1838,33 @@ static void gemm_w_launch(const GemmParams& g, int bm, unsigned grid, hipStream_
   else gemm_w_launch<UP, kBM / 16>(g, grid, s);
 }
 
-// Rows per M-chunk of the bf16 GEMMs: the fewest (32, 64, 160) that hold a group of the mean
-// size plus three standard deviations of a uniform routing.  A chunk's padding rows cost token-row
-// traffic (L2 -> LDS) and MFMAs next to the weight stream; a group split in two costs a second
-// pass over its weights.  Layer, H=2560 E=256 I=1024 k=8, 160 -> 64 -> 32 rows: T=40 (mean 1.25)
-// 549 -> 521 -> 509 us, T=1024 (mean 32) 842 -> 803 -> 890 us.
-static int chunk_rows(int T, int k, int E) {
+// Rows per M-chunk: the fewest that hold a group of the mean size plus two standard deviations
+// of a uniform routing (bf16: 32, 64, 160; int4: 16, 32, 64, 160).  A chunk's padding rows cost
+// token-row traffic (L2 -> LDS) and MFMAs next to the weight stream; a group split in two costs a
+// second pass over its weights (int4: and over their dequantisation).  Measured at H=2560 E=256
+// I=1024 k=8, us per block call with chunks of 16 / 32 / 64 / 160 rows (int4 with the shared expert
+// in launches of its own):
+//   bf16  T=100 (mean 3)   708 /  707 /  707 /  723     int4  T=128  (mean 4)   363 /  372 /  424 / 698
+//         T=603 (mean 19)  926 /  788 /  794 /  822           T=400  (mean 12)  416 /  380 /  430 / 709
+//         T=1536 (mean 48)   - / 1067 /  849 /  876           T=1536 (mean 48)  972 /  649 /  493 / 739
+//         T=2048 (mean 64)   - / 1188 /  973 /  901           T=2048 (mean 64)    - /  781 /  633 / 749
+//                                                             T=3072 (mean 96)    - / 1075 /  832 / 779
+// so int4 groups of up to two 64-row chunks take those too (mean 70), and every size where no
+// 160-row int4 kernel but the register-staged one takes the shape.
+static int chunk_rows(int T, int k, int E, bool q4, bool q4_wide) {
   const float mean = (float)T * (float)k / (float)E;
-  const float want = mean + 3.0f * sqrtf(mean);
-  return want <= 32.0f ? 32 : want <= 64.0f ? 64 : kBM;
+  const float want = mean + 2.0f * sqrtf(mean);
+  if (q4 && want <= 16.0f) return 16;
+  if (want <= 32.0f) return 32;
+  return want <= 64.0f || (q4 && (mean <= 70.0f || !q4_wide)) ? 64 : kBM;
+}
+
+template <bool UP, bool QR>
+static void gemm_q_launch(const GemmParams& g, int bm, unsigned grid, hipStream_t s) {
+  const dim3 gd(grid), bd(64 * kPW);
+  if (bm == 16) hipLaunchKernelGGL((k_grouped_gemm_q<UP, QR, 1>), gd, bd, 0, s, g);
+  else if (bm == 32) hipLaunchKernelGGL((k_grouped_gemm_q<UP, QR, 2>), gd, bd, 0, s, g);
+  else hipLaunchKernelGGL((k_grouped_gemm_q<UP, QR, 4>), gd, bd, 0, s, g);
 }
 
 int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t* ids64, const float* wf,
@@ -1515,19 +1893,31 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
     const char* e = getenv("TMOE_PREFILL_GEMM");
     return e && !strcmp(e, "frag");
   }();
+  // The fragment-load persistent kernel takes K in whole cycles of kPR stages (H and I multiples of
+  // 512); shapes that no tiled kernel takes run on the register-staged one (64 and 128 columns).
+  const int kcyc = kBK * kPR;
+  const bool persistent = H % kcyc == 0 && I % kcyc == 0 && I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32;
   // Whole-line kernel: 128 activation columns (up) or 256 output columns (down) per tile.
   const bool line = I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32 && gemm_w_stages(H / kBK, true) &&
                     gemm_w_stages(I / kBK, true);
-  int bm = q4 || frag || !line ? kBM : chunk_rows(T, k, E);
+  // Small-group int4 kernel: the same tiles, at least kQB stages of 128.
+  const bool qline = I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32 && H / kQK >= kQB && I / kQK >= kQB;
+  int bm = frag || (q4 ? !qline || (has_sh && !line) : !line) ? kBM : chunk_rows(T, k, E, q4 != 0, persistent && H >= 2 * kcyc);
   if (bm != kBM) {
     // More chunks than the descriptor region holds (T k / 64): the router logits' region, read
     // for the last time by the top-k launch, takes them.
-    const size_t chunks = (size_t)T * k / bm + (size_t)n_groups + T / bm + 2;
+    const size_t hit = (size_t)T * k < (size_t)E ? (size_t)T * k : (size_t)E;
+    const size_t chunks = (size_t)T * k / bm + hit + T / (bm < kQShared ? bm : kQShared) + 2;
     if (16 * chunks <= sizeof(float) * (size_t)T * (E + 1)) desc = ws_ptr<int4>(ws, L.logits);
     else bm = kBM;
   }
+  // Int4 groups in chunks of at most 32 rows: the shared expert runs inside the routed launches, where
+  // its K takes four-stage cycles (with 64-row chunks, whose many shared tiles run as fast by
+  // themselves, it gets launches of its own: T=700 388 us against 409, T=1024 457 against 441).
+  const bool fuse = q4 && has_sh && bm <= 32 && H % (4 * kBK) == 0 && I % (4 * kBK) == 0;
+  const int bms = fuse ? kQShared : q4 && bm != kBM ? 64 : bm;
   if (int st = dispatch_launch(ids32, ids64, T, k, E, has_sh ? T : 0, offsets, perm, inv, tile_start, err, s,
-                               desc, bm))
+                               desc, bm, bms))
     return st;
 
   const long mbound = (long)T * k / kBM + (long)(E < T * k ? E : T * k) + (has_sh ? (T + kBM - 1) / kBM : 0) + 1;
@@ -1535,12 +1925,6 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
 
   // One GEMM over groups [lo, hi): bf16 weights, or int4 routed weights (the shared
   // group, always bf16, then gets a launch of its own).
-  // The persistent kernel takes K in whole cycles of kPR stages (H and I multiples of 512),
-  // covers 128 activation columns (up) or 256 output columns (down) per tile and addresses
-  // A rows with 32-bit byte offsets; other shapes take the register-staged kernel (64 and
-  // 128 columns).
-  const int kcyc = kBK * kPR;
-  const bool persistent = H % kcyc == 0 && I % kcyc == 0 && I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32;
   static int n_cu[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return TMOE_ERR_HIP;
@@ -1556,7 +1940,8 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
     // after requesting them, so an up GEMM it would run over K < 2 kPR stages (H = 512) runs
     // on the register-staged kernel instead, with its narrower tiles.
     const bool frag_kernel = routed_q4 || frag;
-    const bool staged = frag_kernel ? !persistent || (g.up && g.K < 2 * kcyc) : !line;
+    const bool small_q = routed_q4 && bm != kBM;
+    const bool staged = small_q ? false : frag_kernel ? !persistent || (g.up && g.K < 2 * kcyc) : !line;
     g.n_ntiles = g.up ? I / (staged ? 64 : kPUpCols) : H / (staged ? 128 : kPDnCols);
     const long grid = (mchunks * g.n_ntiles + 7) / 8 * 8;
     if (staged) {
@@ -1566,6 +1951,9 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
         hipLaunchKernelGGL((k_grouped_gemm<kRing, true>), dim3((unsigned)grid), dim3(256), 0, s, g);
       else
         hipLaunchKernelGGL((k_grouped_gemm<kRing, false>), dim3((unsigned)grid), dim3(256), 0, s, g);
+    } else if (small_q) {
+      if (g.up) qr ? gemm_q_launch<true, true>(g, bm, 2 * pgrid, s) : gemm_q_launch<true, false>(g, bm, 2 * pgrid, s);
+      else qr ? gemm_q_launch<false, true>(g, bm, 2 * pgrid, s) : gemm_q_launch<false, false>(g, bm, 2 * pgrid, s);
     } else if (routed_q4 && qr) {
       hipLaunchKernelGGL((k_grouped_gemm_p<true, true>), dim3(pgrid), dim3(64 * kPW), 0, s, g);
     } else if (routed_q4) {
@@ -1573,9 +1961,9 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
     } else if (frag) {
       hipLaunchKernelGGL((k_grouped_gemm_p<false>), dim3(pgrid), dim3(64 * kPW), 0, s, g);
     } else if (g.up) {
-      gemm_w_launch<true>(g, bm, pgrid, s);
+      gemm_w_launch<true>(g, bms, pgrid, s);
     } else {
-      gemm_w_launch<false>(g, bm, pgrid, s);
+      gemm_w_launch<false>(g, bms, pgrid, s);
     }
   };
   GemmParams up{};
@@ -1588,10 +1976,18 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
   dn.a = act; dn.K = I; dn.gather = 0; dn.up = 0; dn.N = H;
   dn.shw0 = sh_down; dn.shw1 = nullptr; dn.out = ch; dn.out_sh = sh;
   if (q4) {
+    if (fuse) {
+      const float sh = (float)((T + kQShared - 1) / kQShared);
+      const float hit = (float)E * (1.0f - powf(1.0f - (float)k / (float)E, (float)T));
+      // Blocks in proportion to the tiles, a shared one (four times the weight bytes) counted as two:
+      // T=256 383 / 346 / 345 / 351 / 370 us counted as 1 / 2 / 3 / 4 / 6, T=400 382 / 363 / 384 / 388 / 404.
+      const int nb = (int)(4.0f * (float)pgrid * sh / (2.0f * sh + hit) + 7.0f) / 8 * 8;
+      up.sh_blocks = dn.sh_blocks = nb < 8 ? 8 : nb > (int)pgrid ? (int)pgrid : nb;
+    }
     gemm(up, 0, E, true, mbound);
-    if (has_sh) gemm(up, E, E + 1, false, mshared);
+    if (has_sh && !fuse) gemm(up, E, E + 1, false, mshared);
     gemm(dn, 0, E, true, mbound);
-    if (has_sh) gemm(dn, E, E + 1, false, mshared);
+    if (has_sh && !fuse) gemm(dn, E, E + 1, false, mshared);
   } else {
     gemm(up, 0, n_groups, false, mbound);
     gemm(dn, 0, n_groups, false, mbound);
@@ -1632,5 +2028,5 @@ extern "C" int tmoe_dispatch(const int64_t* ids, int T, int k, int E, int32_t* o
   const Ws L = ws_layout(T, 8, E, 8, k, 0);
   if (ws_bytes < L.scratch + sizeof(int32_t) * (size_t)(E + 64)) return TMOE_ERR_WORKSPACE;
   return dispatch_launch(nullptr, ids, T, k, E, 0, offsets, perm, inv, ws_ptr<int32_t>(workspace, L.scratch),
-                         ws_ptr<uint32_t>(workspace, L.status) + kStatusError, (hipStream_t)stream, nullptr, kBM);
+                         ws_ptr<uint32_t>(workspace, L.status) + kStatusError, (hipStream_t)stream, nullptr, kBM, kBM);
 }

@@ -1,11 +1,11 @@
-"""The prefill GEMMs' chunk sizes: groups of 1, 31, 32, 33, 64 and 65 rows through 32- and 64-row chunks
-(the rule takes the fewest rows that hold a mean group plus three standard deviations), at widths that
+"""The prefill GEMMs' chunk sizes: groups of 1, 31, 32, 33, 64 and 65 rows through 16- to 64-row chunks
+(the rule takes the fewest rows that hold a mean group plus two standard deviations), at widths that
 take four or five weight stages per cycle, against the oracle's chain at the bf16 bars."""
 import numpy as np
 import pytest
 import torch
 
-from oracle import moe
+from oracle import bf16, moe
 from tarfa_amd import moe as tm
 from tarfa_amd import seeded
 from tarfa_amd.moe import MoEShape, Workspace
@@ -41,7 +41,7 @@ def test_bf16_chunk_edges(gpu, H, I, E):
 
 @pytest.mark.parametrize("T", [17, 90, 200])
 def test_bf16_chunks_with_shared_expert(gpu, T):
-    """Mean groups of 4, 22 and 50 rows (32-, 64- and 160-row chunks), the shared expert in the same chunks."""
+    """Mean groups of 4, 22 and 50 rows (32- and 64-row chunks), the shared expert in the same chunks."""
     shape = MoEShape(768, 16, 768, 4, 768)
     layer = seeded.make_layer(shape, T, device=gpu)
     ws = Workspace(shape, gpu, tokens=T)
@@ -55,4 +55,60 @@ def test_bf16_chunks_with_shared_expert(gpu, T):
     ref = moe.add_bf16(moe.experts_prefill(f32(x), ids, f32(w), gu, dn, 16),
                        moe.shared_expert(f32(x), *[f32(t) for t in layer.shared]))
     assert_close_bf16(f32(out), ref, f"T={T}")
+    ws.status()
+
+
+def _q4(layer, rows, gpu):
+    """(table, dequantised gate_up and down per expert) of the layer in int4."""
+    parts = []
+    for w in (layer.gate_up, layer.down):
+        q, s = tm.quantize_int4(w)
+        if rows:
+            s = s.float().amax(-1).to(torch.float16)           # one scale per row
+        parts += [q, s.contiguous()]
+    deq = []
+    for q, s in (parts[:2], parts[2:]):
+        q = q.cpu().numpy()
+        n = np.stack([q & 15, q >> 4], axis=-1).reshape(*q.shape[:-1], -1).astype(np.float32) - 8.0
+        s = s.float().cpu().numpy()
+        s = s[..., None] if rows else np.repeat(s, 128, axis=-1)
+        deq.append(bf16.to_f32(bf16.bits(n * s)))
+    table = (tm.expert_table_q4_rows if rows else tm.expert_table_q4)(*parts)
+    return parts, table, dict(enumerate(deq[0])), dict(enumerate(deq[1]))
+
+
+@pytest.mark.parametrize("rows", [False, True])
+@pytest.mark.parametrize("H,I,E", [(512, 512, 40), (768, 640, 40), (512, 640, 16), (768, 512, 16), (768, 640, 6)])
+def test_int4_chunk_edges(gpu, H, I, E, rows):
+    """Means of 6, 14 and 38 rows: 16-, 32- and 64-row chunks; K of 4 (the fewest), 5 and 6 stages."""
+    shape = MoEShape(H, E, I, 1, 0)
+    layer = seeded.make_layer(shape, H + E, device=gpu)
+    parts, table, gu, dn = _q4(layer, rows, gpu)
+    ids = _ids(E, H)
+    T = len(ids)
+    ws = Workspace(shape, gpu, tokens=T)
+    x = seeded.make_tokens(shape, H + E, T, device=gpu)
+    w = torch.linspace(0.1, 1.0, T, device=gpu).to(torch.bfloat16)[:, None].contiguous()
+    out = tm.experts_forward(shape, x, torch.from_numpy(ids).to(gpu), w, table, ws)
+    assert_close_bf16(f32(out), moe.experts_prefill(f32(x), ids, f32(w), gu, dn, E), f"H={H} I={I} E={E}")
+    ws.status()
+
+
+@pytest.mark.parametrize("rows", [False, True])
+@pytest.mark.parametrize("T,I", [(2, 512), (33, 512), (90, 512), (200, 512), (33, 640), (900, 640)])
+def test_int4_chunks_with_shared_expert(gpu, T, I, rows):
+    """Mean groups of 0.5 to 225 rows; the shared expert's tiles inside the int4 launches (I = 512, up to
+    32-row chunks) or in launches of their own."""
+    shape = MoEShape(768, 16, I, 4, I)
+    layer = seeded.make_layer(shape, T, device=gpu)
+    parts, table, gu, dn = _q4(layer, rows, gpu)
+    ws = Workspace(shape, gpu, tokens=T)
+    x = seeded.make_tokens(shape, T, T, device=gpu)
+    logits = seeded.make_logits(shape, T, T, device=gpu)
+    out, ids, w = tm.moe_block(shape, x, table, ws, logits=logits, shared=layer.shared)
+    ids = ids.cpu().numpy()
+    assert np.array_equal(ids, moe.router_topk(logits.cpu().numpy(), 4)[0])
+    ref = moe.add_bf16(moe.experts_prefill(f32(x), ids, f32(w), gu, dn, 16),
+                       moe.shared_expert(f32(x), *[f32(t) for t in layer.shared]))
+    assert_close_bf16(f32(out), ref, f"T={T} I={I}")
     ws.status()
