@@ -19,7 +19,8 @@ and for decode calls the route-reuse counters (``routing_telemetry()``, recorded
 the device).  Device-detected errors (an expert id outside [0, E], an expired
 bounded wait) are polled without stalling the compute stream: after every call (every
 ``status_poll`` calls, default 1) the workspace status word is copied to pinned host
-memory on a side stream, and the next call that finds the copy landed raises
+memory (decode calls: on their own stream; prefill calls: on a side stream), and the next call
+that finds the copy landed raises
 ``RuntimeError`` if it is set -- at the latest the first call after the engine's next
 synchronisation point (the reference synchronises after every call,
 tarfa/engine/fused_int4.py:203-204).  ``check_status()`` is the synchronous check.
@@ -62,6 +63,7 @@ class _CallBook:
         self.status_poll = int(status_poll)
         self._status_host = torch.zeros(1, dtype=torch.int32, pin_memory=True)
         self._status_event = None
+        self._inline_event = torch.cuda.Event()  # at most one copy is outstanding, so its event is reused
         self._side = None
         _BOOKS.add(self)
 
@@ -71,13 +73,21 @@ class _CallBook:
             code = -7 if flags & 2 else -6      # TMOE_ERR_TIMEOUT / TMOE_ERR_EXPERT_ID
             check(code, "libtmoe device status (asynchronous poll)")
 
-    def _poll(self, stream):
+    def _poll(self, stream, inline):
         ev = self._status_event
         if ev is not None and ev.query():
             self._status_event = None
             self._raise_if_flagged(int(self._status_host[0]))
         total = self.counts["decode"] + self.counts["prefill"]
         if self.status_poll > 0 and self._status_event is None and total % self.status_poll == 0:
+            # Decode calls copy the word on their own stream: a 1.5 us copy there, where the fork to a
+            # side stream (a wait, an event, a stream switch) took half of a small decode call's ~79 us
+            # of host time.  Longer calls keep it off the compute stream.
+            if inline:
+                self._status_host.copy_(self.workspace.status_word, non_blocking=True)
+                self._inline_event.record(stream)
+                self._status_event = self._inline_event
+                return
             if self._side is None:
                 self._side = torch.cuda.Stream(self.device)
             buf = self.workspace.buf
@@ -111,7 +121,7 @@ class _CallBook:
     def call(self, kind, fn, record_ids=None):
         """Run fn() (one libtmoe launch sequence on the current stream) as a ``kind`` call."""
         stream = torch.cuda.current_stream(self.device)
-        self._poll(stream)
+        self._poll(stream, kind == "decode")
         if self.timing:
             e0 = self._event()
             e0.record(stream)

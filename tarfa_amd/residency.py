@@ -36,7 +36,7 @@ import torch
 
 from . import seeded
 from ._lib import check, lib
-from .moe import MoEShape, quantize_int4
+from .moe import MoEShape, _stream, quantize_int4
 
 
 def part_shapes(shape: MoEShape, int4: bool):
@@ -355,7 +355,7 @@ class RouteTelemetry:
         """Record one token's routing for every layer (ids [L, k] int64 on the device)."""
         ids = self.ids if ids is None else ids
         st = lib().tmoe_route_record(ids.data_ptr(), self.L, self.k, self.E, self.state.data_ptr(),
-                                     self.state.numel(), torch.cuda.current_stream(ids.device).cuda_stream)
+                                     self.state.numel(), _stream(ids.device))
         check(st, "tmoe_route_record")
 
     def counters(self):
