@@ -37,82 +37,83 @@ __global__ __launch_bounds__(256) void k_router_logits(const uint16_t* __restric
 }
 
 // The same logits for many tokens as a GEMM on the matrix cores: v_mfma_f32_16x16x32_bf16
-// (exact bf16 products, fp32 accumulation).  Block (tb, eb) of 4 waves computes tokens
-// 32 tb .. + 31 x experts 32 eb .. + 31 (four 16 x 16 blocks); the K steps (32 wide) are
+// (exact bf16 products, fp32 accumulation).  Block (tb, eb) of 4 waves computes 16 TA tokens x
+// 16 TB experts (TA TB 16 x 16 blocks); the K steps (32 wide) are
 // dealt round-robin to the 4 waves (step s to wave s % 4), and the waves' partial sums are
-// added through LDS in wave order, so each logit is one fixed-order fp32 sum.  Operand
-// fragments come straight from memory, lane l holding row l % 16 and k = 8 (l / 16) .. + 7
-// of a step (16 bytes), for the token rows (A) and the router rows (B); rows past T or E
-// repeat the last one and are never stored.  The GEMV form above reads the whole router
+// added through LDS in wave order, so each logit is one fixed-order fp32 sum (the same at every
+// tile size).  Operand fragments come straight from memory, lane l holding row l % 16 and
+// k = 8 (l / 16) .. + 7 of a step (16 bytes), for the token rows (A) and the router rows (B); rows
+// past T or E repeat the last one and are never stored.  The GEMV form above reads the whole router
 // weight once per token (1.3 GB of L2 reads per 1000 tokens at H = 2560, E = 256); this
-// reads it once per 32 tokens.  H a multiple of 32.
+// reads it once per 16 TA tokens, and the tokens once per 16 TB experts.  H a multiple of 32.
+// Bound by that L2 traffic: TA x TB of 2 x 2 reads 335 MB at T = 4096, 4 x 4 164 MB.
 typedef __bf16 rt_bf16x8 __attribute__((ext_vector_type(8)));
-constexpr int kRtUnroll = 8;   // k steps of a wave whose loads are issued together
+template <int TA, int TB>
 __global__ __launch_bounds__(256) void k_router_logits_mfma(const uint16_t* __restrict__ x,
                                                             const uint16_t* __restrict__ wg, int T, int H, int E,
                                                             float* __restrict__ logits) {
-  __shared__ f32x4 red[4][4][64];   // [wave][block (i, j)][lane]
+  constexpr int kUnroll = TA + TB <= 4 ? 8 : 4;   // k steps of a wave whose loads are issued together
+  __shared__ f32x4 red[4][TA * TB][64];   // [wave][block (i, j)][lane]
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int t0 = (int)blockIdx.x * 32, e0 = (int)blockIdx.y * 32;
+  const int t0 = (int)blockIdx.x * 16 * TA, e0 = (int)blockIdx.y * 16 * TB;
   const int r = lane & 15, kq = (lane >> 4) * 8;
-  const uint16_t* pa[2];
-  const uint16_t* pb[2];
+  const uint16_t* pa[TA];
+  const uint16_t* pb[TB];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    pa[i] = x + (size_t)min(t0 + 16 * i + r, T - 1) * H + kq;
-    pb[i] = wg + (size_t)min(e0 + 16 * i + r, E - 1) * H + kq;
-  }
-  f32x4 c[2][2];
+  for (int i = 0; i < TA; ++i) pa[i] = x + (size_t)min(t0 + 16 * i + r, T - 1) * H + kq;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int j = 0; j < TB; ++j) pb[j] = wg + (size_t)min(e0 + 16 * j + r, E - 1) * H + kq;
+  f32x4 c[TA][TB];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) c[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto step = [&](const u32x4 (&a)[2], const u32x4 (&b)[2]) {
+  for (int i = 0; i < TA; ++i)
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < TB; ++j) c[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](const u32x4 (&a)[TA], const u32x4 (&b)[TB]) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+    for (int i = 0; i < TA; ++i)
+#pragma unroll
+      for (int j = 0; j < TB; ++j)
         c[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(rt_bf16x8, a[i]),
                                                           __builtin_bit_cast(rt_bf16x8, b[j]), c[i][j], 0, 0, 0);
   };
+  auto load = [&](u32x4 (&a)[TA], u32x4 (&b)[TB], int st) {
+#pragma unroll
+    for (int i = 0; i < TA; ++i) a[i] = ld16(pa[i] + 32 * st);
+#pragma unroll
+    for (int j = 0; j < TB; ++j) b[j] = ld16(pb[j] + 32 * st);
+  };
   const int nsteps = H / 32;
   int st = wid;
-  for (; st + 4 * (kRtUnroll - 1) < nsteps; st += 4 * kRtUnroll) {
-    u32x4 a[kRtUnroll][2], b[kRtUnroll][2];
+  for (; st + 4 * (kUnroll - 1) < nsteps; st += 4 * kUnroll) {
+    u32x4 a[kUnroll][TA], b[kUnroll][TB];
 #pragma unroll
-    for (int u = 0; u < kRtUnroll; ++u)
+    for (int u = 0; u < kUnroll; ++u) load(a[u], b[u], st + 4 * u);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        a[u][i] = ld16(pa[i] + 32 * (st + 4 * u));
-        b[u][i] = ld16(pb[i] + 32 * (st + 4 * u));
-      }
-#pragma unroll
-    for (int u = 0; u < kRtUnroll; ++u) step(a[u], b[u]);
+    for (int u = 0; u < kUnroll; ++u) step(a[u], b[u]);
   }
   for (; st < nsteps; st += 4) {
-    u32x4 a[2], b[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      a[i] = ld16(pa[i] + 32 * st);
-      b[i] = ld16(pb[i] + 32 * st);
-    }
+    u32x4 a[TA], b[TB];
+    load(a, b, st);
     step(a, b);
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < TA; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) red[wid][2 * i + j][lane] = c[i][j];
+    for (int j = 0; j < TB; ++j) red[wid][i * TB + j][lane] = c[i][j];
   __syncthreads();
-  // Wave w stores block (i, j) = (w / 2, w % 2): lane l holds tokens 16 i + 4 (l / 16) + q,
+  // Wave w stores blocks (i, j) = w, w + 4, ...: lane l holds tokens 16 i + 4 (l / 16) + q,
   // expert 16 j + l % 16.
-  const int i = wid >> 1, j = wid & 1;
-  const f32x4 v = ((red[0][wid][lane] + red[1][wid][lane]) + red[2][wid][lane]) + red[3][wid][lane];
-  const int e = e0 + 16 * j + r;
-  if (e < E) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int t = t0 + 16 * i + 4 * (lane >> 4) + q;
-      if (t < T) logits[(size_t)t * E + e] = v[q];
+  for (int b = wid; b < TA * TB; b += 4) {
+    const int i = b / TB, j = b % TB;
+    const f32x4 v = ((red[0][b][lane] + red[1][b][lane]) + red[2][b][lane]) + red[3][b][lane];
+    const int e = e0 + 16 * j + r;
+    if (e < E) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int t = t0 + 16 * i + 4 * (lane >> 4) + q;
+        if (t < T) logits[(size_t)t * E + e] = v[q];
+      }
     }
   }
 }
@@ -141,8 +142,15 @@ int launch_router_logits(const uint16_t* x, const uint16_t* wg, int T, int H, in
     return e ? atoi(e) : kRouterMfmaFrom;
   }();
   if (T >= mfma_from && H % 32 == 0) {
-    const dim3 g((T + 31) / 32, (E + 31) / 32);
-    hipLaunchKernelGGL(k_router_logits_mfma, g, dim3(256), 0, s, x, wg, T, H, E, logits);
+    // The largest tile that still leaves a block for each of 256 CUs.
+    auto blocks = [&](int ta, int tb) { return ((T + 16 * ta - 1) / (16 * ta)) * ((E + 16 * tb - 1) / (16 * tb)); };
+    auto grid = [&](int ta, int tb) { return dim3((T + 16 * ta - 1) / (16 * ta), (E + 16 * tb - 1) / (16 * tb)); };
+    if (blocks(4, 4) >= 256)
+      hipLaunchKernelGGL((k_router_logits_mfma<4, 4>), grid(4, 4), dim3(256), 0, s, x, wg, T, H, E, logits);
+    else if (blocks(4, 2) >= 256)
+      hipLaunchKernelGGL((k_router_logits_mfma<4, 2>), grid(4, 2), dim3(256), 0, s, x, wg, T, H, E, logits);
+    else
+      hipLaunchKernelGGL((k_router_logits_mfma<2, 2>), grid(2, 2), dim3(256), 0, s, x, wg, T, H, E, logits);
     return hipGetLastError() == hipSuccess ? TMOE_OK : TMOE_ERR_HIP;
   }
   const int nc = (H + 511) / 512;
