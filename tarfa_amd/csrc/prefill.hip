@@ -188,6 +188,80 @@ __global__ __launch_bounds__(1024) void k_dispatch_scatter(const int32_t* ids32,
   }
 }
 
+// Both of the above in one launch for few entries (T k <= 1024, one per thread; T = 12: 10.1 us in two
+// launches of ~5 us, each mostly start-up and one pass over the ids).  Every expert's entries are
+// marked in a bitmask in LDS indexed by j = slot T + t; the counts are its popcounts and an entry's
+// place among its expert's is the popcount before it, so the order is the stable one.
+constexpr int kSmallN = 1024, kSmallWords = 1 << 14;
+// Words per expert, odd: thread e's walk over expert e's words meets no bank conflicts.
+__host__ __device__ inline int small_stride(int n) { return ((n + 31) / 32) | 1; }
+__global__ __launch_bounds__(1024) void k_dispatch_small(const int32_t* ids32, const int64_t* ids64, int T, int k,
+                                                         int E, int shared_rows, int32_t* offsets, int32_t* perm,
+                                                         int32_t* inv, int32_t* tile_start, uint32_t* err, int4* desc,
+                                                         int bm, int bms) {
+  __shared__ uint32_t mask[kSmallWords];
+  __shared__ int sc[1024], sk[1024], wave_c[16], wave_k[16];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int n = T * k, nw = (n + 31) / 32, stride = small_stride(n);
+  int e = -1, j = 0;
+  if (tid < n) {
+    e = load_id(ids32, ids64, tid);
+    const int t = tid / k;
+    j = (tid - t * k) * T + t;
+    if (e < 0 || e >= E) {
+      if (e != E && err) atomicOr(err, 1u);
+      e = -1;
+      inv[tid] = -1;
+    }
+  }
+  for (int w = tid; w < E * stride; w += 1024) mask[w] = 0u;
+  __syncthreads();
+  if (e >= 0) atomicOr(&mask[e * stride + (j >> 5)], 1u << (j & 31));
+  __syncthreads();
+  int c = 0;
+  if (tid < E)
+    for (int w = 0; w < nw; ++w) c += __popc(mask[tid * stride + w]);
+  const int ch = tid < E ? (c + bm - 1) / bm : (tid == E ? (shared_rows + bms - 1) / bms : 0);
+  // Inclusive scans of counts and M-chunks (groups 0..E-1, then the shared group).
+  int ic = c, ik = ch;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int a = __shfl_up(ic, d), b = __shfl_up(ik, d);
+    if (lane >= d) {
+      ic += a;
+      ik += b;
+    }
+  }
+  if (lane == 63) {
+    wave_c[wid] = ic;
+    wave_k[wid] = ik;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    ic += w < wid ? wave_c[w] : 0;
+    ik += w < wid ? wave_k[w] : 0;
+  }
+  sc[tid] = ic;
+  sk[tid] = ik;
+  if (tid < E) offsets[tid + 1] = ic;
+  if (tid == 0) { offsets[0] = 0; tile_start[0] = 0; }
+  if (tid <= E) tile_start[tid + 1] = ik;
+  __syncthreads();
+  if (e >= 0) {
+    int r = e ? sc[e - 1] : 0;
+    for (int w = 0; w < (j >> 5); ++w) r += __popc(mask[e * stride + w]);
+    r += __popc(mask[e * stride + (j >> 5)] & ((1u << (j & 31)) - 1u));
+    perm[r] = tid;
+    inv[tid] = r;
+  }
+  // Group tid's descriptors.
+  const bool shared = tid == E && shared_rows > 0;
+  if (!desc || !(tid < E || shared)) return;
+  const int rows = shared ? shared_rows : c, gm = shared ? bms : bm, first = shared ? 0 : ic - c;
+  for (int m = 0; m < ch; ++m) desc[ik - ch + m] = int4{tid, min(gm, rows - m * gm), first + m * gm, 0};
+}
+
 // ---------------------------------------------------------------- grouped GEMM
 struct GemmParams {
   const uint16_t* a;         // up: x [T, H]; down: act [(T*k + T), I]
@@ -1808,6 +1882,11 @@ int dispatch_launch(const int32_t* ids32, const int64_t* ids64, int T, int k, in
                     int32_t* offsets, int32_t* perm, int32_t* inv, int32_t* tile_start, uint32_t* err,
                     hipStream_t s, int4* desc, int bm, int bms) {
   if ((long)T * k > kScatterMaxN) return TMOE_ERR_SHAPE;
+  if (T * k <= kSmallN && E * small_stride(T * k) <= kSmallWords) {
+    hipLaunchKernelGGL(k_dispatch_small, dim3(1), dim3(1024), 0, s, ids32, ids64, T, k, E, shared_rows, offsets, perm,
+                       inv, tile_start, err, desc, bm, bms);
+    return hipGetLastError() == hipSuccess ? TMOE_OK : TMOE_ERR_HIP;
+  }
   hipLaunchKernelGGL(k_dispatch_count, dim3(1), dim3(1024), 0, s, ids32, ids64, T, k, E, shared_rows, offsets,
                      tile_start, inv, err, desc, bm, bms);
   hipLaunchKernelGGL(k_dispatch_scatter, dim3(E), dim3(1024), 0, s, ids32, ids64, T, k, offsets, perm, inv);

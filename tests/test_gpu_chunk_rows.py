@@ -112,3 +112,20 @@ def test_int4_chunks_with_shared_expert(gpu, T, I, rows):
                        moe.shared_expert(f32(x), *[f32(t) for t in layer.shared]))
     assert_close_bf16(f32(out), ref, f"T={T} I={I}")
     ws.status()
+
+
+@pytest.mark.parametrize("T,E,k", [(1, 8, 8), (64, 256, 16), (128, 495, 8), (128, 497, 8), (129, 256, 8), (33, 1023, 4),
+                                   (1024, 3, 1), (1025, 3, 1)])
+def test_dispatch_one_launch_bounds(gpu, T, E, k):
+    """T k and E around the limits of the one-launch dispatch (1024 entries, 16384 mask words), with sentinels."""
+    ids = np.random.default_rng(T * E).integers(0, E + 1, (T, k)).astype(np.int64)     # E: the sentinel
+    ws = Workspace(MoEShape(128, E, 64, k if k <= E else E), gpu, tokens=T)
+    offsets, perm, inv = tm.dispatch(torch.from_numpy(ids).to(gpu), E, ws)
+    o_ref, p_ref = moe.dispatch(ids, E)
+    n = int(o_ref[-1])
+    assert np.array_equal(offsets.cpu().numpy(), o_ref)
+    assert np.array_equal(perm.cpu().numpy()[:n], p_ref)
+    inv_ref = np.full(T * k, -1, np.int64)
+    inv_ref[p_ref] = np.arange(n)
+    assert np.array_equal(inv.cpu().numpy(), inv_ref)
+    ws.status()
