@@ -1,7 +1,7 @@
 // Prefill (T > 1) MoE layer: dispatch, MFMA grouped GEMMs, expert-ascending combine.
 //
 //   dispatch  histogram + exclusive scan (1 block), stable per-expert compaction
-//             (1 block per expert) -> offsets, perm (expert, slot, token order), inv,
+//             (1 block per expert; few entries: both in one block) -> offsets, perm (expert, slot, token order), inv,
 //             and the grouped-GEMM tile schedule.      tarfa/engine/fused_int4.py:228-229, 241
 //   up GEMM   per group: [rows x H] . [H x 2I] on v_mfma_f32_16x16x32_bf16, epilogue
 //             act = bf16(bf16(silu(bf16 g)) * bf16 u)    fused_int4.py:242-243
@@ -1462,9 +1462,12 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
 //   4 g + s of the stage's 256-byte rows (the same permutation of k for both operands).
 //   A: global -> LDS, 4 rows x 256 bytes per load, row r's chunk c at chunk c ^ (r % 16); a ring of
 //   kQB + 1 slots requested kQB stages ahead, as the weights (in registers).
-// What bounds it is the dequantisation (~23 VALU instructions per 8 weights and lane) beside the
-// weight stream, so two blocks share a CU (128 registers a wave): one block's waits and epilogues
-// overlap the other's arithmetic.
+// What bounds it is the dequantisation (19 VALU instructions per 8 weights and lane, ~92 cycles per
+// fragment against 16 of each MFMA) beside the weight stream, so two blocks share a CU (128 registers
+// a wave): one block's waits and epilogues overlap the other's arithmetic.  H=2560 E=256 I=1024 k=8,
+// routed launches, k_grouped_gemm_p -> this: T=603 561 -> ~270 us (1.01 GB, 3.7 TB/s), T=12 249 -> 104
+// (with the shared expert inside; 344 MB).  Six stages in flight were slower (T=12 call 185 -> 204 us,
+// T=603 337 -> 344), as were 64-row chunks with eight and one block per CU (T=603 383 -> 413).
 // The stages of a block's tiles form one stream: stage sc of a tile requests stage sc + kQB, the next
 // tile's first ones past the tile's end.  A tile may have any number of stages >= kQB: a tile's row
 // indices are fetched two tiles ahead, at least kQB stage waits before they are used.

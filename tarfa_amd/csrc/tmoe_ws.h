@@ -75,7 +75,8 @@ struct Ws {
   size_t inv;      // int32[T * k]
   size_t scratch;  // int32[E + 64]      dispatch counters
   size_t ch;       // bf16[T * k * H]    per-assignment expert outputs, unscaled (T > 1)
-  size_t desc;     // int32x4[T * k / 64 + E + T / 64 + 2]   prefill M-chunk descriptors (T > 1)
+  size_t desc;     // int32x4[T * k / 64 + E + T / 64 + 2]   prefill M-chunk descriptors (T > 1; chunks of
+                   // fewer than 160 rows, more of them, lie in the logits region once the top-k has run)
   size_t xn;       // bf16[T * H]        RMSNorm of the hidden state (the layer entry points)
   size_t sbord;    // small-batch combine order: int32 rows[kSbMaxEntries], f32 weights[kSbMaxEntries],
                    // int32 counts[kSbMaxTokens]; then the down kernel's slice descriptors
