@@ -1140,8 +1140,8 @@ __device__ __forceinline__ void gemm_w_body(const GemmParams& p, int bid, int nb
   u32x4* const reg = lB + wid * kWReg;
   // The stage's 8-row parts are loads 0 .. 2 MB - 1 over the waves; a wave whose load index lies
   // past them repeats an earlier part (the same bytes to the same place).
-  auto a_part = [](int x) { return MB == 1 ? (x & 1) : x < 2 * MB ? x : x - kPW / 2; };
-  static_assert(MB == 1 || (2 * MB) % kPW == 0 || (2 * MB) % kPW == kPW / 2, "repeats are earlier parts");
+  auto a_part = [](int x) { return x < 2 * MB ? x : x - kPW / 2; };
+  static_assert((2 * MB) % kPW == 0 || (2 * MB) % kPW == kPW / 2, "repeats are earlier parts");
 
   const int c_lo = sload1(p.tile_start + p.group_lo);
   const int c_hi = sload1(p.tile_start + p.group_hi);
