@@ -1984,7 +1984,8 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
                     gemm_w_stages(I / kBK, true);
   // Small-group int4 kernel: the same tiles, at least kQB stages of 128.
   const bool qline = I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32 && H / kQK >= kQB && I / kQK >= kQB;
-  int bm = frag || (q4 ? !qline || (has_sh && !line) : !line) ? kBM : chunk_rows(T, k, E, q4 != 0, persistent && H >= 2 * kcyc);
+  const bool tiled = !frag && (q4 ? qline && (!has_sh || line) : line);
+  int bm = tiled ? chunk_rows(T, k, E, q4 != 0, persistent && H >= 2 * kcyc) : kBM;
   if (bm != kBM) {
     // More chunks than the descriptor region holds (T k / 64): the router logits' region, read
     // for the last time by the top-k launch, takes them.
