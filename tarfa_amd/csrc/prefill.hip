@@ -649,6 +649,11 @@ __device__ __forceinline__ void gld4_into(uint32_t& v, const void* sbase, uint32
 __device__ __forceinline__ void gld2_into(uint32_t& v, const void* sbase, uint32_t voff) {
   asm volatile("global_load_ushort %0, %1, %2" : "+v"(v) : "v"(voff), "s"(sbase));
 }
+// Facts about the paths that run, as comments in the assembly for the check of these loads there
+// (tests/test_asm_pipeline.py): PATH_COUNT counts passes of NAME, PATH_FACT says how many there are when
+// this place is reached (">= n" or "== n"; the count restarts).
+#define PATH_COUNT(NAME) asm volatile("; path + " NAME)
+#define PATH_FACT(NAME, CMP, N) asm volatile("; path " NAME " " CMP " %0" : : "n"(N))
 // 16 bytes per lane from global memory straight into LDS at lds + 16 lane (M0 = lds).
 // Nothing else in the kernel uses M0.
 __device__ __forceinline__ void gdma16(const void* sbase, uint32_t voff, const void* lds) {
@@ -1050,6 +1055,7 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_p(GemmParams p) {
   // tile: its own first stages again, never multiplied).  K / 64 is a multiple of kPR, so
   // tiles start on a cycle boundary and every load is unconditional.
   auto cycle = [&](int st0, auto tail_tag) {
+    PATH_COUNT("cycle");
     constexpr bool kTail = decltype(tail_tag)::value;   // the tile's last cycle
 #pragma unroll
     for (int u = 0; u < kPR; ++u) {
@@ -1076,12 +1082,14 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_p(GemmParams p) {
       stage_end();
     }
   };
+  PATH_COUNT("cycle");
   for (int j = 0; j < ntile; ++j) {
     for (int st0 = 0; st0 < nk - kPR; st0 += kPR) cycle(st0, std::false_type{});
     // The next tile's perm entries were fetched before this tile's first stage: the
     // nk - kPR >= kPR stage waits since then leave only the last kPA - 1 stages' loads
     // outstanding.  (A gathering launch therefore needs K >= 2 kPR stages; the host sends
     // K = 512 gathers to the register-staged kernel.)
+    PATH_FACT("cycle", ">=", 2);   // the last tile's last (or the prologue), and this one's before it
     a_offsets(a_off_nxt, pv_nxt, nxt);
     cycle(nk - kPR, std::true_type{});
     if (p.up) epilogue(cur, std::true_type{});
@@ -1375,12 +1383,14 @@ __device__ __forceinline__ void gemm_w_body(const GemmParams& p, int bid, int nb
       // places past the pass) redirected to the sink: the next tile's first waits count them.
 #pragma unroll 1
       for (int q = 0; q < NST; ++q) {
+        PATH_COUNT("store");
         const int x = tid + q * 64 * kPW;
         const int rr = x / CPR, qc = x - rr * CPR, row = P * RPP + rr;
         const u32x4 v = *reinterpret_cast<const u32x4*>(rowp(rr) + ((qc ^ (2 * ((rr >> 2) & 3))) * 16));
         const bool ok = x < RPP * CPR && row < t.m;
         *reinterpret_cast<u32x4*>(ok ? t.o + (size_t)row * p.N + qc * 8 : p.sink) = v;
       }
+      PATH_FACT("store", "==", NST);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       barrier_raw();
     }
@@ -1660,6 +1670,7 @@ __device__ __forceinline__ void gemm_q_body(const GemmParams& p, int bid, int nb
     static_assert(n < 64, "vmcnt range");
     wait_vmcnt<n>();
     barrier_raw();
+    PATH_COUNT("stage");
   };
   // Epilogue through the A slot that the tile's last stage used (no load targets it until the next
   // stage): row r's 16-byte chunk q at chunk q ^ 2 ((r / 4) % 4); C fragment lane l holds rows
@@ -1747,6 +1758,7 @@ __device__ __forceinline__ void gemm_q_body(const GemmParams& p, int bid, int nb
         nxt = tile(j + 1);
         // The next tile's row indices and this one's row scales were requested at the previous
         // tile's start, at least kQB stages ago.
+        PATH_FACT("stage", ">=", kQB);
         wait_fetched();
 #pragma unroll
         for (int q = 0; q < kALoads; ++q) a_off_cur[q] = a_off_nxt[q];
