@@ -1170,21 +1170,21 @@ __device__ __forceinline__ void gemm_w_body(const GemmParams& p, int bid, int nb
     const bool shared = g == p.E;
     PTile t;
     t.m = d.y;
-    t.gather = p.up && !shared;
-    t.arow0 = (!p.up && shared ? p.shared_row0 : 0) + row0;
-    const int c0 = p.up ? nt * kPUpCols + wid * 16 : nt * kPDnCols + wid * 32;
-    if (p.up) t.o = p.out + (size_t)(shared ? p.shared_row0 + row0 : row0) * p.N + nt * kPUpCols;
+    t.gather = UP && !shared;
+    t.arow0 = (!UP && shared ? p.shared_row0 : 0) + row0;
+    const int c0 = UP ? nt * kPUpCols + wid * 16 : nt * kPDnCols + wid * 32;
+    if (UP) t.o = p.out + (size_t)(shared ? p.shared_row0 + row0 : row0) * p.N + nt * kPUpCols;
     else t.o = (shared ? p.out_sh : p.out) + (size_t)row0 * p.N + nt * kPDnCols;
     const uint16_t *w0, *w1;
     if (shared) {
       w0 = p.shw0;
-      w1 = p.up ? p.shw1 : p.shw0;
+      w1 = UP ? p.shw1 : p.shw0;
     } else {
-      w0 = w1 = reinterpret_cast<const uint16_t*>(sload_ptr(p.table + 2 * g + (p.up ? 0 : 1)));
+      w0 = w1 = reinterpret_cast<const uint16_t*>(sload_ptr(p.table + 2 * g + (UP ? 0 : 1)));
     }
 #pragma unroll
     for (int nb = 0; nb < kPNB; ++nb) {
-      const int wr = p.up ? ((nb && !shared) ? p.I : 0) + c0 : c0 + 16 * nb;
+      const int wr = UP ? ((nb && !shared) ? p.I : 0) + c0 : c0 + 16 * nb;
       t.b[nb] = (nb ? w1 : w0) + (size_t)wr * K;
       t.q[nb] = nullptr;
       t.sc[nb] = nullptr;
@@ -1223,19 +1223,25 @@ __device__ __forceinline__ void gemm_w_body(const GemmParams& p, int bid, int nb
   u32x4 breg[kWB][kWBLoads];
   const int nk = K / kBK;   // a multiple of kWB, at least 2 kWB
   uint32_t a_off_cur[kALoads], a_off_nxt[kALoads];
-  uint32_t pv_cur[kALoads], pv_nxt[kALoads];
-  // Always kALoads loads (tiles without a gather read perm[0]): the waits count them.
+  uint32_t pv_cur[kALoads], pv_nxt[kALoads];   // up only
+  // Up: always kALoads loads (the shared group, not gathered, reads perm[0]): the waits count them.
+  constexpr int kPerm = UP ? kALoads : 0;
   auto fetch_perm = [&](uint32_t* pv, const PTile& t) {
-    const int32_t* pp = p.perm + (t.gather ? t.arow0 : 0);
+    if constexpr (UP) {
+      const int32_t* pp = p.perm + (t.gather ? t.arow0 : 0);
 #pragma unroll
-    for (int j = 0; j < kALoads; ++j) pv[j] = gld4(pp, t.gather ? (uint32_t)(min(a_row[j], t.m - 1) * 4) : 0u);
+      for (int j = 0; j < kALoads; ++j) pv[j] = gld4(pp, t.gather ? (uint32_t)(min(a_row[j], t.m - 1) * 4) : 0u);
+    }
   };
   auto a_offsets = [&](uint32_t* o, uint32_t* pv, const PTile& t) {
+    if constexpr (UP) {
 #pragma unroll
-    for (int j = 0; j < kALoads; ++j) asm volatile("" : "+v"(pv[j]));
+      for (int j = 0; j < kALoads; ++j) asm volatile("" : "+v"(pv[j]));
+    }
 #pragma unroll
     for (int j = 0; j < kALoads; ++j) {
-      const int row = t.gather ? (int)pv[j] / p.k : t.arow0 + min(a_row[j], t.m - 1);
+      int row = t.arow0 + min(a_row[j], t.m - 1);
+      if constexpr (UP) row = t.gather ? (int)pv[j] / p.k : row;
       o[j] = (uint32_t)row * (uint32_t)(K * 2) + (uint32_t)(a_col * 2);
     }
   };
@@ -1262,13 +1268,13 @@ __device__ __forceinline__ void gemm_w_body(const GemmParams& p, int bid, int nb
   // operations of an epilogue in between).  The registers pass through the asm, so nothing
   // reads them before the wait.
   // Stores per thread in one epilogue; the first kWB iterations of the next tile add them and
-  // the next tile's perm loads (kXH) to their waits.
+  // the next tile's perm loads (up; kXH) to their waits.
   constexpr int kEpiBlocks = MB <= 4 ? MB : MB / 2;         // 16-row blocks per epilogue pass
   constexpr int kEpiPasses = MB / kEpiBlocks;
   constexpr int kRowChunks = (UP ? kPUpCols : kPDnCols) / 8;   // 16-byte pieces of an output row
   constexpr int kPassStores = (16 * kEpiBlocks * kRowChunks + 64 * kPW - 1) / (64 * kPW);
   constexpr int kEpiStores = kPassStores * kEpiPasses;
-  constexpr int kXH = kEpiStores + kALoads;
+  constexpr int kXH = kEpiStores + kPerm;
   auto wait_b = [&](int bs, bool head) {
     constexpr int n = (kWB - 1) * kWOps + kALoads;
     static_assert(kWBLoads == 4 && n + kXH < 64, "four weight registers per stage; vmcnt range");

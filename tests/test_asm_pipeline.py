@@ -184,13 +184,25 @@ def test_checker_path_facts():
     assert early_uses([l.replace("vmcnt(2)", "vmcnt(3)") for l in least]) == [(load, body[7])]
 
 
-@pytest.mark.skipif(not shutil.which(B.HIPCC) and not os.path.exists(B.HIPCC), reason="hipcc not installed")
-def test_grouped_gemm_pipeline_loads_untouched_before_a_wait(tmp_path):
-    out = tmp_path / "prefill.s"
+@pytest.fixture(scope="module")
+def asm(tmp_path_factory):
+    if not shutil.which(B.HIPCC) and not os.path.exists(B.HIPCC):
+        pytest.skip("hipcc not installed")
+    out = tmp_path_factory.mktemp("asm") / "prefill.s"
     r = subprocess.run([B.HIPCC, *B.CFLAGS, "--cuda-device-only", "-S", os.path.join(B.CSRC, "prefill.hip"),
                         "-o", str(out)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
-    asm = out.read_text()
+    return out.read_text()
+
+
+def test_grouped_gemms_use_no_scratch(asm):
+    """A spilled register is reloaded behind a vmcnt(0), which drains the stages in flight."""
+    sizes = dict(re.findall(r"\.set (_ZN4tmoe\d+k_grouped_gemm\w*)\.private_seg_size, (\d+)", asm))
+    assert any("gemm_w" in n for n in sizes), sizes
+    assert not {n: s for n, s in sizes.items() if int(s)}
+
+
+def test_grouped_gemm_pipeline_loads_untouched_before_a_wait(asm):
     names = re.findall(r"^(_ZN4tmoe\d+k_grouped_gemm\w*):", asm, re.M)
     for kernel in ("gemm_pI", "gemm_wI", "gemm_qI"):
         assert any(kernel in n for n in names), (kernel, names)

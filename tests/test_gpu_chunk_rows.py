@@ -39,10 +39,11 @@ def test_bf16_chunk_edges(gpu, H, I, E):
     ws.status()
 
 
-@pytest.mark.parametrize("T", [17, 90, 200])
-def test_bf16_chunks_with_shared_expert(gpu, T):
-    """Mean groups of 4, 22 and 50 rows (32- and 64-row chunks), the shared expert in the same chunks."""
-    shape = MoEShape(768, 16, 768, 4, 768)
+@pytest.mark.parametrize("T,I", [(17, 768), (90, 768), (200, 768), (4096, 640)])
+def test_bf16_chunks_with_shared_expert(gpu, T, I):
+    """Mean groups of 4, 22, 50 and 1024 rows, the shared expert in the same chunks; the last in 160-row
+    chunks whose down GEMM takes five-stage cycles."""
+    shape = MoEShape(768, 16, I, 4, I)
     layer = seeded.make_layer(shape, T, device=gpu)
     ws = Workspace(shape, gpu, tokens=T)
     x = seeded.make_tokens(shape, T, T, device=gpu)
