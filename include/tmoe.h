@@ -287,6 +287,18 @@ int tmoe_route_record(const int64_t* ids, int L, int k, int E, void* state, size
  */
 int tmoe_debug_decode_trace(void* buf, size_t bytes);
 
+/* What the prefill path (T > 1, past the small-batch kernels) launches for a shape, computed on the
+ * host without a device; no counterpart in the reference.  q4: 0 bf16, 1 int4 with group scales, 2
+ * with row scales; blocks: the device's compute units, a multiple of 8; counts: E host ints, the
+ * rows of each expert (bf16: the chunk size depends on them; NULL: the smallest it may take).
+ * plan[0], plan[1]: rows per M-chunk, routed experts and shared expert; plan[2]: 1 where the shared
+ * expert runs inside the int4 launches; plan[3]: 1 where the whole-line bf16 and small-group int4
+ * kernels take the shape; plan[4]: the workspace byte where a call leaves the bf16 GEMMs' rows per
+ * chunk (int32).
+ */
+int tmoe_debug_prefill_plan(int T, int H, int E, int I, int k, int Is, int q4, int blocks,
+                            const int32_t* counts, int64_t* plan);
+
 #ifdef __cplusplus
 }
 #endif

@@ -43,14 +43,105 @@ __device__ __forceinline__ bool ids_aligned(const int32_t* ids32, const int64_t*
   return ((ids32 ? (uintptr_t)ids32 : (uintptr_t)ids64) & 15u) == 0;
 }
 
+// ---------------------------------------------------------------- rows per M-chunk, bf16
+// The dispatch chooses the rows per chunk of the bf16 GEMMs (32, 64 or 160; one size for all groups)
+// from the group sizes, which the host does not know.  A smaller chunk stages and multiplies less
+// padding; a group cut into more of them has its weights read (from L2 or the infinity cache) and
+// staged more often.  In units of 1/100 of the time in which every block multiplies one 32-row tile:
+//   a group's first chunk    285  300  320   (32, 64, 160 rows; its weights come from HBM)
+//   each further one          90  100  200
+//   but a round of tiles     100  112  230   and tiles take whole rounds of the launch's blocks.
+// Fitted to us per call with the size forced, 120 runs of 8 shapes, T = 17 .. 4096, uniform, Zipf and
+// one-set-of-experts routings.  At H=2560 E=256 I=1024 k=8, 32 / 64 / 160 rows:
+//   T=603  uniform 751 /  758 / 793   Zipf  774 / 768 / 791   every token the same experts 214 / 159 / 182
+//   T=1024         874 /  780 / 817         908 / 817 / 827                                320 / 228 / 216
+//   T=2048        1162 /  932 / 871        1170 / 968 / 957                                599 / 409 / 369
+// The size it names is within 0.3 % of the fastest one on average, 5.4 % at most, and within 0.3 % of 160
+// rows or faster but for two cases (1.5 %: 257 us against 254).
+struct ChunkRule {
+  int lo = 0;                       // smallest size to choose among (32 or 64; 0: the size is given)
+  float H, I;                       // K of the up and of the down launch
+  float up_rounds, dn_rounds;       // rounds of the launches' blocks that one chunk's column tiles take
+};
+constexpr int kRowSizes[3] = {32, 64, kBM};
+// The size to take, where `hit` groups have rows and n[s] chunks of size s hold them.
+__host__ __device__ inline int chunk_pick(const ChunkRule& r, int hit, const int (&n)[3]) {
+  constexpr float first[3] = {285.f, 300.f, 320.f}, further[3] = {90.f, 100.f, 200.f}, turn[3] = {100.f, 112.f, 230.f};
+  float cost[3];
+  for (int s = 0; s < 3; ++s) {
+    const float work = (first[s] * (float)hit + further[s] * (float)(n[s] - hit)) *
+                       (r.up_rounds * r.H + r.dn_rounds * r.I);
+    const float rounds = turn[s] * (ceilf((float)n[s] * r.up_rounds) * r.H + ceilf((float)n[s] * r.dn_rounds) * r.I);
+    cost[s] = work > rounds ? work : rounds;
+  }
+  return r.lo == 32 && cost[0] <= cost[1] && cost[0] <= cost[2] ? 32 : cost[1] <= cost[2] ? 64 : kBM;
+}
+
 // ---------------------------------------------------------------- dispatch
+// The rows per chunk of a launch: bm of the routed groups, bms of the shared one; where rule.lo names a
+// size, both are chosen from the counts.  `out` (or null) takes the bf16 GEMM's size, bms.
+struct ChunkRows {
+  int bm, bms;
+  ChunkRule rule;
+  int32_t* out;
+};
+// Inclusive scans over a block of 1024 threads, one group each, of the groups' rows (c) and of their
+// M-chunks (v).  Where the size is to be chosen, v holds 16 bits each of the chunks of 32, 64 and 160
+// rows and of the groups that have any (at most 33,792, at T k = 2^19), so the totals of one scan
+// decide and the chosen field is the scan.
+struct GroupScan {
+  int c, v;        // inclusive, this thread's group
+  int bm, bms;     // rows per chunk
+};
+__device__ __forceinline__ GroupScan scan_groups(const ChunkRows& r, int E, int rows, int shared_rows, int* wave_c,
+                                                 unsigned long long* wave_v) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int m = tid < E ? rows : tid == E ? shared_rows : 0;
+  int c = tid < E ? rows : 0;
+  unsigned long long v;
+  if (r.rule.lo)
+    v = (unsigned)((m + 31) / 32) | (unsigned)((m + 63) / 64) << 16 |
+        ((unsigned long long)((m + kBM - 1) / kBM) << 32) | ((unsigned long long)(m > 0) << 48);
+  else
+    v = (unsigned)(tid < E ? (m + r.bm - 1) / r.bm : (m + r.bms - 1) / r.bms);
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int a = __shfl_up(c, d);
+    const unsigned long long b = __shfl_up(v, d);
+    if (lane >= d) {
+      c += a;
+      v += b;
+    }
+  }
+  if (lane == 63) {
+    wave_c[wid] = c;
+    wave_v[wid] = v;
+  }
+  __syncthreads();
+  unsigned long long all = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    c += w < wid ? wave_c[w] : 0;
+    v += w < wid ? wave_v[w] : 0;
+    all += wave_v[w];
+  }
+  GroupScan g{c, (int)v, r.bm, r.bms};
+  if (r.rule.lo) {
+    const int n[3] = {(int)(all & 0xffff), (int)(all >> 16 & 0xffff), (int)(all >> 32 & 0xffff)};
+    g.bm = g.bms = chunk_pick(r.rule, (int)(all >> 48), n);
+    g.v = (int)(v >> (g.bm == 32 ? 0 : g.bm == 64 ? 16 : 32) & 0xffff);
+  }
+  if (r.out && tid == 0) *r.out = g.bms;
+  return g;
+}
+
 // One block of 1024 threads: per-expert counts, offsets, M-chunk schedule, inv := -1, and
 // (desc non-null) one descriptor per M-chunk (bm rows, the shared
 // group's bms): {group, rows, first row in group order, 0}.
 __global__ __launch_bounds__(1024) void k_dispatch_count(const int32_t* ids32, const int64_t* ids64, int T, int k,
                                                          int E, int shared_rows, int32_t* offsets,
                                                          int32_t* tile_start, int32_t* inv, uint32_t* err,
-                                                         int4* desc, int bm, int bms) {
+                                                         int4* desc, ChunkRows rows_arg) {
   __shared__ int cnt[1024];
   const int tid = threadIdx.x;
   for (int e = tid; e < 1024; e += 1024) cnt[e] = 0;
@@ -85,25 +176,16 @@ __global__ __launch_bounds__(1024) void k_dispatch_count(const int32_t* ids32, c
   }
   if (bad && err) atomicOr(err, 1u);
   __syncthreads();
-  // Inclusive Hillis-Steele scans of counts and M-chunks (groups 0..E-1, then the shared group).
-  const int c = tid < E ? cnt[tid] : 0;
-  int ch = tid < E ? (c + bm - 1) / bm : (tid == E ? (shared_rows + bms - 1) / bms : 0);
-  __shared__ int sc[1024], sk[1025];
-  sc[tid] = c;
-  sk[tid] = ch;
-  if (tid == 0) sk[1024] = 0;
-  __syncthreads();
-  for (int d = 1; d < 1024; d <<= 1) {
-    const int a = tid >= d ? sc[tid - d] : 0;
-    const int b = tid >= d ? sk[tid - d] : 0;
-    __syncthreads();
-    sc[tid] += a;
-    sk[tid] += b;
-    __syncthreads();
-  }
-  if (tid < E) offsets[tid + 1] = sc[tid];
+  __shared__ int sc[1024], sk[1024], wave_c[16];
+  __shared__ unsigned long long wave_v[16];
+  const GroupScan g0 = scan_groups(rows_arg, E, cnt[tid], shared_rows, wave_c, wave_v);
+  const int bm = g0.bm, bms = g0.bms;
+  sc[tid] = g0.c;
+  sk[tid] = g0.v;
+  if (tid < E) offsets[tid + 1] = g0.c;
   if (tid == 0) { offsets[0] = 0; tile_start[0] = 0; }
-  if (tid <= E) tile_start[tid + 1] = sk[tid];
+  if (tid <= E) tile_start[tid + 1] = g0.v;
+  __syncthreads();
   if (!desc) return;
   // M-chunk mt of group g (sk[g - 1] <= mt < sk[g]): rows r0 = (mt - sk[g - 1]) gm onwards.
   const int n_groups = shared_rows > 0 ? E + 1 : E;
@@ -198,10 +280,11 @@ __host__ __device__ inline int small_stride(int n) { return ((n + 31) / 32) | 1;
 __global__ __launch_bounds__(1024) void k_dispatch_small(const int32_t* ids32, const int64_t* ids64, int T, int k,
                                                          int E, int shared_rows, int32_t* offsets, int32_t* perm,
                                                          int32_t* inv, int32_t* tile_start, uint32_t* err, int4* desc,
-                                                         int bm, int bms) {
+                                                         ChunkRows rows_arg) {
   __shared__ uint32_t mask[kSmallWords];
-  __shared__ int sc[1024], sk[1024], wave_c[16], wave_k[16];
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  __shared__ int sc[1024], wave_c[16];
+  __shared__ unsigned long long wave_v[16];
+  const int tid = threadIdx.x;
   const int n = T * k, nw = (n + 31) / 32, stride = small_stride(n);
   int e = -1, j = 0;
   if (tid < n) {
@@ -221,32 +304,12 @@ __global__ __launch_bounds__(1024) void k_dispatch_small(const int32_t* ids32, c
   int c = 0;
   if (tid < E)
     for (int w = 0; w < nw; ++w) c += __popc(mask[tid * stride + w]);
-  const int ch = tid < E ? (c + bm - 1) / bm : (tid == E ? (shared_rows + bms - 1) / bms : 0);
-  // Inclusive scans of counts and M-chunks (groups 0..E-1, then the shared group).
-  int ic = c, ik = ch;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int a = __shfl_up(ic, d), b = __shfl_up(ik, d);
-    if (lane >= d) {
-      ic += a;
-      ik += b;
-    }
-  }
-  if (lane == 63) {
-    wave_c[wid] = ic;
-    wave_k[wid] = ik;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int w = 0; w < 16; ++w) {
-    ic += w < wid ? wave_c[w] : 0;
-    ik += w < wid ? wave_k[w] : 0;
-  }
-  sc[tid] = ic;
-  sk[tid] = ik;
-  if (tid < E) offsets[tid + 1] = ic;
+  const GroupScan g0 = scan_groups(rows_arg, E, c, shared_rows, wave_c, wave_v);
+  const int bm = g0.bm, bms = g0.bms;
+  sc[tid] = g0.c;
+  if (tid < E) offsets[tid + 1] = g0.c;
   if (tid == 0) { offsets[0] = 0; tile_start[0] = 0; }
-  if (tid <= E) tile_start[tid + 1] = ik;
+  if (tid <= E) tile_start[tid + 1] = g0.v;
   __syncthreads();
   if (e >= 0) {
     int r = e ? sc[e - 1] : 0;
@@ -258,8 +321,9 @@ __global__ __launch_bounds__(1024) void k_dispatch_small(const int32_t* ids32, c
   // Group tid's descriptors.
   const bool shared = tid == E && shared_rows > 0;
   if (!desc || !(tid < E || shared)) return;
-  const int rows = shared ? shared_rows : c, gm = shared ? bms : bm, first = shared ? 0 : ic - c;
-  for (int m = 0; m < ch; ++m) desc[ik - ch + m] = int4{tid, min(gm, rows - m * gm), first + m * gm, 0};
+  const int rows = shared ? shared_rows : c, gm = shared ? bms : bm, first = shared ? 0 : g0.c - c;
+  const int ch = (rows + gm - 1) / gm;
+  for (int m = 0; m < ch; ++m) desc[g0.v - ch + m] = int4{tid, min(gm, rows - m * gm), first + m * gm, 0};
 }
 
 // ---------------------------------------------------------------- grouped GEMM
@@ -279,6 +343,7 @@ struct GemmParams {
   uint16_t* out;             // up: act; down: ch [T*k, H], each expert output unscaled
   uint16_t* out_sh;          // down: sh [T, H], the shared expert's output before its gate
   const int4* desc;          // persistent kernel: M-chunk descriptors {group, rows, first row, 0}
+  const int32_t* rows;       // whole-line kernel: rows per chunk (one word)
   int sh_blocks;             // int4 small-group launch: blocks that run the shared group's (bf16) tiles
   uint16_t* sink;            // 16 bytes nobody reads: whole-line kernel stores of rows past a tile
 };
@@ -1134,7 +1199,8 @@ constexpr int kWLdsB = kPW * kWReg;              // and of the wave regions
 
 // Block bid of nblk walking groups [p.group_lo, p.group_hi).
 template <bool UP, int WB, int MB>
-__device__ __forceinline__ void gemm_w_body(const GemmParams& p, int bid, int nblk, u32x4* const lA, u32x4* const lB) {
+__device__ __forceinline__ void gemm_w_body(const GemmParams& p, int c_lo, int c_hi, int bid, int nblk,
+                                            u32x4* const lA, u32x4* const lB) {
   constexpr int kWB = WB, kWA = WB, kWAS = WB + 1;
   constexpr int kSlot = MB * 16 * 8;             // u32x4 per A slot (16 MB rows x 128 B)
   constexpr int kALoads = (2 * MB + kPW - 1) / kPW;   // A loads per wave per stage
@@ -1151,8 +1217,6 @@ __device__ __forceinline__ void gemm_w_body(const GemmParams& p, int bid, int nb
   auto a_part = [](int x) { return x < 2 * MB ? x : x - kPW / 2; };
   static_assert((2 * MB) % kPW == 0 || (2 * MB) % kPW == kPW / 2, "repeats are earlier parts");
 
-  const int c_lo = sload1(p.tile_start + p.group_lo);
-  const int c_hi = sload1(p.tile_start + p.group_hi);
   const int total = (c_hi - c_lo) * p.n_ntiles;
   const int nbx = nblk >> 3;
   const int xcd = bid & 7, qb = bid >> 3;
@@ -1299,16 +1363,31 @@ __device__ __forceinline__ void gemm_w_body(const GemmParams& p, int bid, int nb
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       const int rd = ks ? rd1 : rd0;
-      bf16x8_t b[kPNB];
+      bf16x8_t b[kPNB], a[4];
 #pragma unroll
       for (int nb = 0; nb < kPNB; ++nb) b[nb] = as_bf16x8(reg[nb * 128 + rd]);
+      // Up, 160 rows: token fragments are read two row blocks before their MFMAs and sched_barrier keeps
+      // them there.  Left to the compiler, some builds wait for each read (T=4096 call 1010 -> 1049 us).
+      constexpr bool kAhead = UP && MB == 10;
       auto blocks = [&](int i0, int i1) {
+        if (kAhead) {
+          a[0] = as_bf16x8(la[i0 * 128 + rd]);
+          a[1] = as_bf16x8(la[(i0 + 1) * 128 + rd]);
+        }
 #pragma unroll
         for (int i = i0; i < i1; ++i) {
-          const bf16x8_t a = as_bf16x8(la[i * 128 + rd]);
+          if (!kAhead) {
+            a[i % 4] = as_bf16x8(la[i * 128 + rd]);
+          } else if (i % 2 == 0) {
+            if (i + 2 < i1) {
+              a[(i + 2) % 4] = as_bf16x8(la[(i + 2) * 128 + rd]);
+              a[(i + 3) % 4] = as_bf16x8(la[(i + 3) * 128 + rd]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
 #pragma unroll
           for (int nb = 0; nb < kPNB; ++nb)
-            acc[i][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[nb], acc[i][nb], 0, 0, 0);
+            acc[i][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i % 4], b[nb], acc[i][nb], 0, 0, 0);
         }
       };
       // Down: chunks of at most 128 rows (about half the groups at ~128 tokens per expert)
@@ -1462,11 +1541,18 @@ __device__ __forceinline__ void gemm_w_body(const GemmParams& p, int bid, int nb
   wait_vmcnt<0>();
 }
 
-template <bool UP, int WB, int MB>
+// The dispatch has chosen the rows per chunk (p.rows), so one launch holds the body of each size; all run
+// one block per CU.  WB: weight stages of 160-row tiles; up tiles of 32 and 64 rows take 4 (five only
+// where K has no cycles of four, which an up GEMM's, a multiple of 256, always has).
+template <bool UP, int WB>
 __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_w(GemmParams p) {
-  __shared__ u32x4 lA[kWLdsA<WB, MB>];
+  constexpr int WS = UP ? 4 : WB;
+  __shared__ u32x4 lA[kWLdsA<WB, kBM / 16>];
   __shared__ u32x4 lB[kWLdsB];
-  gemm_w_body<UP, WB, MB>(p, (int)blockIdx.x, (int)gridDim.x, lA, lB);
+  const int rows = sload1(p.rows), c_lo = sload1(p.tile_start + p.group_lo), c_hi = sload1(p.tile_start + p.group_hi);
+  if (rows == 32) gemm_w_body<UP, WS, 2>(p, c_lo, c_hi, (int)blockIdx.x, (int)gridDim.x, lA, lB);
+  else if (rows == 64) gemm_w_body<UP, WS, 4>(p, c_lo, c_hi, (int)blockIdx.x, (int)gridDim.x, lA, lB);
+  else gemm_w_body<UP, WB, kBM / 16>(p, c_lo, c_hi, (int)blockIdx.x, (int)gridDim.x, lA, lB);
 }
 
 // ---------------------------------------------------------------- grouped GEMM, int4, small groups
@@ -1790,9 +1876,8 @@ __global__ __launch_bounds__(64 * kPW, 4) void k_grouped_gemm_q(GemmParams p) {
   __shared__ u32x4 lds[MB >= 4 || kQLds<MB> > kShLds ? kQLds<MB> : kShLds];
   if (MB < 4 && (int)blockIdx.x < p.sh_blocks) {   // 64-row chunks: never beside the shared group
     if constexpr (MB < 4) {
-      p.group_lo = p.E;
-      p.group_hi = p.E + 1;
-      gemm_w_body<UP, 4, kQShared / 16>(p, (int)blockIdx.x, p.sh_blocks, lds, lds + kWLdsA<4, kQShared / 16>);
+      gemm_w_body<UP, 4, kQShared / 16>(p, sload1(p.tile_start + p.E), sload1(p.tile_start + p.E + 1), (int)blockIdx.x,
+                                        p.sh_blocks, lds, lds + kWLdsA<4, kQShared / 16>);
     }
   } else {
     gemm_q_body<UP, QR, MB>(p, (int)blockIdx.x - p.sh_blocks, (int)gridDim.x - p.sh_blocks, lds);
@@ -1901,22 +1986,22 @@ __global__ __launch_bounds__(256) void k_combine(const int32_t* ids32, const int
 // ---------------------------------------------------------------- driver
 int dispatch_launch(const int32_t* ids32, const int64_t* ids64, int T, int k, int E, int shared_rows,
                     int32_t* offsets, int32_t* perm, int32_t* inv, int32_t* tile_start, uint32_t* err,
-                    hipStream_t s, int4* desc, int bm, int bms) {
+                    hipStream_t s, int4* desc, const ChunkRows& rows) {
   if ((long)T * k > kScatterMaxN) return TMOE_ERR_SHAPE;
   if (T * k <= kSmallN && E * small_stride(T * k) <= kSmallWords) {
     hipLaunchKernelGGL(k_dispatch_small, dim3(1), dim3(1024), 0, s, ids32, ids64, T, k, E, shared_rows, offsets, perm,
-                       inv, tile_start, err, desc, bm, bms);
+                       inv, tile_start, err, desc, rows);
     return hipGetLastError() == hipSuccess ? TMOE_OK : TMOE_ERR_HIP;
   }
   hipLaunchKernelGGL(k_dispatch_count, dim3(1), dim3(1024), 0, s, ids32, ids64, T, k, E, shared_rows, offsets,
-                     tile_start, inv, err, desc, bm, bms);
+                     tile_start, inv, err, desc, rows);
   hipLaunchKernelGGL(k_dispatch_scatter, dim3(E), dim3(1024), 0, s, ids32, ids64, T, k, offsets, perm, inv);
   return hipGetLastError() == hipSuccess ? TMOE_OK : TMOE_ERR_HIP;
 }
 
 // The whole-line bf16 kernel's weight stages in registers for a K of nk stages: 4 or 5, whichever
-// divides nk with at least two cycles per tile, 0 if neither.  Where both do: 5 for the up GEMM of
-// 160-row chunks (655 -> 646 us at T=4096), else 4 (with 32- and 64-row chunks, whose smaller
+// divides nk with at least two cycles per tile, 0 if neither.  Where both do: 5 for the up GEMM
+// (160-row tiles: 655 -> 646 us at T=4096), else 4 (with 32- and 64-row tiles, whose smaller
 // accumulators leave room for 8, four stages were faster: T=40 layer 509 us against 520, T=1024
 // 803 against 810, H=2560 E=256 I=1024 k=8).
 static int gemm_w_stages(int nk, bool five_first) {
@@ -1924,39 +2009,28 @@ static int gemm_w_stages(int nk, bool five_first) {
   return five && (five_first || !four) ? 5 : four ? 4 : 0;
 }
 
-template <bool UP, int MB>
-static void gemm_w_launch(const GemmParams& g, unsigned grid, hipStream_t s) {
-  if (gemm_w_stages(g.K / kBK, UP && MB == kBM / 16) == 5)
-    hipLaunchKernelGGL((k_grouped_gemm_w<UP, 5, MB>), dim3(grid), dim3(64 * kPW), 0, s, g);
-  else
-    hipLaunchKernelGGL((k_grouped_gemm_w<UP, 4, MB>), dim3(grid), dim3(64 * kPW), 0, s, g);
-}
 template <bool UP>
-static void gemm_w_launch(const GemmParams& g, int bm, unsigned grid, hipStream_t s) {
-  if (bm == 32) gemm_w_launch<UP, 2>(g, grid, s);
-  else if (bm == 64) gemm_w_launch<UP, 4>(g, grid, s);
-  else gemm_w_launch<UP, kBM / 16>(g, grid, s);
+static void gemm_w_launch(const GemmParams& g, unsigned grid, hipStream_t s) {
+  if (gemm_w_stages(g.K / kBK, UP) == 5)
+    hipLaunchKernelGGL((k_grouped_gemm_w<UP, 5>), dim3(grid), dim3(64 * kPW), 0, s, g);
+  else
+    hipLaunchKernelGGL((k_grouped_gemm_w<UP, 4>), dim3(grid), dim3(64 * kPW), 0, s, g);
 }
 
-// Rows per M-chunk: the fewest that hold a group of the mean size plus two standard deviations
-// of a uniform routing (bf16: 32, 64, 160; int4: 16, 32, 64, 160).  A chunk's padding rows cost
-// token-row traffic (L2 -> LDS) and MFMAs next to the weight stream; a group split in two costs a
-// second pass over its weights (int4: and over their dequantisation).  Measured at H=2560 E=256
-// I=1024 k=8, us per block call with chunks of 16 / 32 / 64 / 160 rows (int4 with the shared expert
-// in launches of its own):
-//   bf16  T=100 (mean 3)   708 /  707 /  707 /  723     int4  T=128  (mean 4)   363 /  372 /  424 / 698
-//         T=603 (mean 19)  926 /  788 /  794 /  822           T=400  (mean 12)  416 /  380 /  430 / 709
-//         T=1536 (mean 48)   - / 1067 /  849 /  876           T=1536 (mean 48)  972 /  649 /  493 / 739
-//         T=2048 (mean 64)   - / 1188 /  973 /  901           T=2048 (mean 64)    - /  781 /  633 / 749
-//                                                             T=3072 (mean 96)    - / 1075 /  832 / 779
-// so int4 groups of up to two 64-row chunks take those too (mean 70), and every size where no
-// 160-row int4 kernel but the register-staged one takes the shape.
-static int chunk_rows(int T, int k, int E, bool q4, bool q4_wide) {
+// Rows per M-chunk of the int4 groups: the fewest of 16, 32, 64 and 160 that hold a group of the mean
+// size plus two standard deviations of a uniform routing.  A chunk's padding rows cost token-row
+// traffic (L2 -> LDS) and MFMAs next to the weight stream; a group split in two costs a second pass
+// over its weights and their dequantisation.  Measured at H=2560 E=256 I=1024 k=8, us per block call
+// with chunks of 16 / 32 / 64 / 160 rows (the shared expert in launches of its own):
+//   T=128  (mean 4)  363 /  372 / 424 / 698     T=1536 (mean 48) 972 /  649 / 493 / 739
+//   T=400  (mean 12) 416 /  380 / 430 / 709     T=2048 (mean 64)   - /  781 / 633 / 749
+//                                               T=3072 (mean 96)   - / 1075 / 832 / 779
+// so groups of up to two 64-row chunks take those too (mean 70), and every size where no 160-row int4
+// kernel but the register-staged one takes the shape (H=2048 E=128 I=768, T=4096: 506 against 691).
+static int chunk_rows_q4(int T, int k, int E, bool q4_wide) {
   const float mean = (float)T * (float)k / (float)E;
   const float want = mean + 2.0f * sqrtf(mean);
-  if (q4 && want <= 16.0f) return 16;
-  if (want <= 32.0f) return 32;
-  return want <= 64.0f || (q4 && (mean <= 70.0f || !q4_wide)) ? 64 : kBM;
+  return want <= 16.0f ? 16 : want <= 32.0f ? 32 : want <= 64.0f || mean <= 70.0f || !q4_wide ? 64 : kBM;
 }
 
 template <bool UP, bool QR>
@@ -1966,6 +2040,54 @@ static void gemm_q_launch(const GemmParams& g, int bm, unsigned grid, hipStream_
   else if (bm == 32) hipLaunchKernelGGL((k_grouped_gemm_q<UP, QR, 2>), gd, bd, 0, s, g);
   else hipLaunchKernelGGL((k_grouped_gemm_q<UP, QR, 4>), gd, bd, 0, s, g);
 }
+
+// What a prefill call of this shape launches; host arithmetic only.
+struct PrefillPlan {
+  bool persistent, line, tiled;   // shapes the fragment-load and the whole-line kernel (and k_grouped_gemm_q) take
+  bool desc_logits;               // M-chunk descriptors in the logits region
+  bool fuse;                      // the shared expert inside the int4 launches
+  int bm, bms;                    // rows per chunk, routed and shared (where rule.lo is 0)
+  ChunkRule rule;                 // bf16: how the dispatch chooses them
+};
+static PrefillPlan prefill_plan(int T, int H, int E, int I, int k, bool has_sh, int q4, bool frag, int blocks) {
+  PrefillPlan p{};
+  // A rows are addressed with 32-bit byte offsets by the persistent kernels.
+  const bool ofs32 = (size_t)T * H * 2 < ((size_t)1 << 32) && ((size_t)T * k + T) * I * 2 < ((size_t)1 << 32);
+  // The fragment-load persistent kernel takes K in whole cycles of kPR stages (H and I multiples of
+  // 512); shapes that no tiled kernel takes run on the register-staged one (64 and 128 columns).
+  const int kcyc = kBK * kPR;
+  p.persistent = H % kcyc == 0 && I % kcyc == 0 && I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32;
+  // Whole-line kernel: 128 activation columns (up) or 256 output columns (down) per tile.
+  p.line = I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32 && gemm_w_stages(H / kBK, true) &&
+           gemm_w_stages(I / kBK, true);
+  // Small-group int4 kernel: the same tiles, at least kQB stages of 128.
+  const bool qline = I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32 && H / kQK >= kQB && I / kQK >= kQB;
+  p.tiled = !frag && (q4 ? qline && (!has_sh || p.line) : p.line);
+  // The smallest chunks the call may use; more of them than the descriptor region holds (T k / 64)
+  // go to the router logits' region, read for the last time by the top-k launch.
+  int bm = kBM;
+  if (p.tiled) bm = q4 ? chunk_rows_q4(T, k, E, p.persistent && H >= 2 * kcyc) : 32;
+  for (; bm != kBM; bm = q4 || bm == 64 ? kBM : 64) {
+    const size_t hit = (size_t)T * k < (size_t)E ? (size_t)T * k : (size_t)E;
+    const size_t chunks = (size_t)T * k / bm + hit + T / (bm < kQShared ? bm : kQShared) + 2;
+    if (16 * chunks <= sizeof(float) * (size_t)T * (E + 1)) break;
+  }
+  p.desc_logits = bm != kBM;
+  // Int4 groups in chunks of at most 32 rows: the shared expert runs inside the routed launches, where
+  // its K takes four-stage cycles (with 64-row chunks, whose many shared tiles run as fast by
+  // themselves, it gets launches of its own: T=700 388 us against 409, T=1024 457 against 441).
+  p.fuse = q4 && has_sh && bm <= 32 && I % (4 * kBK) == 0;
+  p.bm = bm;
+  p.bms = p.fuse ? kQShared : q4 && bm != kBM ? 64 : bm;
+  if (!q4 && bm != kBM)
+    p.rule = ChunkRule{bm, (float)H, (float)I, (float)(I / kPUpCols) / blocks, (float)(H / kPDnCols) / blocks};
+  return p;
+}
+
+// The word that tells the whole-line kernel its rows per chunk, and 16 bytes nobody reads before it:
+// both past tile_start's E + 2 words.
+static int sink_word(int E) { return (E + 5) & ~3; }
+static int rows_word(int E) { return sink_word(E) + 4; }
 
 int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t* ids64, const float* wf,
                    const uint16_t* wb, const uint64_t* table, const uint16_t* sh_gate, const uint16_t* sh_up,
@@ -1985,40 +2107,23 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
   uint16_t* act = ws_ptr<uint16_t>(ws, L.act);
   uint16_t* ch = ws_ptr<uint16_t>(ws, L.ch);
   uint16_t* sh = ws_ptr<uint16_t>(ws, L.sh);
-  int4* desc = ws_ptr<int4>(ws, L.desc);
   const int n_groups = has_sh ? E + 1 : E;
-  // A rows are addressed with 32-bit byte offsets by the persistent kernels.
-  const bool ofs32 = (size_t)T * H * 2 < ((size_t)1 << 32) && ((size_t)T * k + T) * I * 2 < ((size_t)1 << 32);
   static const bool frag = [] {
     const char* e = getenv("TMOE_PREFILL_GEMM");
     return e && !strcmp(e, "frag");
   }();
-  // The fragment-load persistent kernel takes K in whole cycles of kPR stages (H and I multiples of
-  // 512); shapes that no tiled kernel takes run on the register-staged one (64 and 128 columns).
-  const int kcyc = kBK * kPR;
-  const bool persistent = H % kcyc == 0 && I % kcyc == 0 && I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32;
-  // Whole-line kernel: 128 activation columns (up) or 256 output columns (down) per tile.
-  const bool line = I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32 && gemm_w_stages(H / kBK, true) &&
-                    gemm_w_stages(I / kBK, true);
-  // Small-group int4 kernel: the same tiles, at least kQB stages of 128.
-  const bool qline = I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32 && H / kQK >= kQB && I / kQK >= kQB;
-  const bool tiled = !frag && (q4 ? qline && (!has_sh || line) : line);
-  int bm = tiled ? chunk_rows(T, k, E, q4 != 0, persistent && H >= 2 * kcyc) : kBM;
-  if (bm != kBM) {
-    // More chunks than the descriptor region holds (T k / 64): the router logits' region, read
-    // for the last time by the top-k launch, takes them.
-    const size_t hit = (size_t)T * k < (size_t)E ? (size_t)T * k : (size_t)E;
-    const size_t chunks = (size_t)T * k / bm + hit + T / (bm < kQShared ? bm : kQShared) + 2;
-    if (16 * chunks <= sizeof(float) * (size_t)T * (E + 1)) desc = ws_ptr<int4>(ws, L.logits);
-    else bm = kBM;
-  }
-  // Int4 groups in chunks of at most 32 rows: the shared expert runs inside the routed launches, where
-  // its K takes four-stage cycles (with 64-row chunks, whose many shared tiles run as fast by
-  // themselves, it gets launches of its own: T=700 388 us against 409, T=1024 457 against 441).
-  const bool fuse = q4 && has_sh && bm <= 32 && H % (4 * kBK) == 0 && I % (4 * kBK) == 0;
-  const int bms = fuse ? kQShared : q4 && bm != kBM ? 64 : bm;
-  if (int st = dispatch_launch(ids32, ids64, T, k, E, has_sh ? T : 0, offsets, perm, inv, tile_start, err, s,
-                               desc, bm, bms))
+  static int n_cu[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return TMOE_ERR_HIP;
+  if (!n_cu[dev] && hipDeviceGetAttribute(&n_cu[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return TMOE_ERR_HIP;
+  const unsigned pgrid = (unsigned)(n_cu[dev] >= 8 ? n_cu[dev] / 8 * 8 : 8);
+  const PrefillPlan pl = prefill_plan(T, H, E, I, k, has_sh, q4, frag, (int)pgrid);
+  const bool persistent = pl.persistent, line = pl.line, fuse = pl.fuse;
+  const int bm = pl.bm, kcyc = kBK * kPR;
+  int4* desc = ws_ptr<int4>(ws, pl.desc_logits ? L.logits : L.desc);
+  if (int st = dispatch_launch(ids32, ids64, T, k, E, has_sh ? T : 0, offsets, perm, inv, tile_start, err, s, desc,
+                               ChunkRows{bm, pl.bms, pl.rule, tile_start + rows_word(E)}))
     return st;
 
   const long mbound = (long)T * k / kBM + (long)(E < T * k ? E : T * k) + (has_sh ? (T + kBM - 1) / kBM : 0) + 1;
@@ -2026,12 +2131,6 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
 
   // One GEMM over groups [lo, hi): bf16 weights, or int4 routed weights (the shared
   // group, always bf16, then gets a launch of its own).
-  static int n_cu[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return TMOE_ERR_HIP;
-  if (!n_cu[dev] && hipDeviceGetAttribute(&n_cu[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return TMOE_ERR_HIP;
-  const unsigned pgrid = (unsigned)(n_cu[dev] >= 8 ? n_cu[dev] / 8 * 8 : 8);
   // bf16 groups run on the whole-line kernel where it takes the shape; TMOE_PREFILL_GEMM=frag
   // selects the fragment-load kernel (int4 groups always use it).
   auto gemm = [&](GemmParams g, int lo, int hi, bool routed_q4, long mchunks) {
@@ -2062,9 +2161,9 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
     } else if (frag) {
       hipLaunchKernelGGL((k_grouped_gemm_p<false>), dim3(pgrid), dim3(64 * kPW), 0, s, g);
     } else if (g.up) {
-      gemm_w_launch<true>(g, bms, pgrid, s);
+      gemm_w_launch<true>(g, pgrid, s);
     } else {
-      gemm_w_launch<false>(g, bms, pgrid, s);
+      gemm_w_launch<false>(g, pgrid, s);
     }
   };
   GemmParams up{};
@@ -2072,7 +2171,8 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
   up.T = T; up.E = E; up.k = k; up.n_groups = n_groups; up.up = 1; up.N = I; up.I = I;
   up.table = table; up.shw0 = sh_gate; up.shw1 = sh_up; up.shared_row0 = T * k; up.out = act;
   up.desc = desc;
-  up.sink = reinterpret_cast<uint16_t*>(tile_start + ((E + 5) & ~3));   // past tile_start's E + 2 words
+  up.sink = reinterpret_cast<uint16_t*>(tile_start + sink_word(E));
+  up.rows = tile_start + rows_word(E);
   GemmParams dn = up;
   dn.a = act; dn.K = I; dn.gather = 0; dn.up = 0; dn.N = H;
   dn.shw0 = sh_down; dn.shw1 = nullptr; dn.out = ch; dn.out_sh = sh;
@@ -2129,5 +2229,33 @@ extern "C" int tmoe_dispatch(const int64_t* ids, int T, int k, int E, int32_t* o
   const Ws L = ws_layout(T, 8, E, 8, k, 0);
   if (ws_bytes < L.scratch + sizeof(int32_t) * (size_t)(E + 64)) return TMOE_ERR_WORKSPACE;
   return dispatch_launch(nullptr, ids, T, k, E, 0, offsets, perm, inv, ws_ptr<int32_t>(workspace, L.scratch),
-                         ws_ptr<uint32_t>(workspace, L.status) + kStatusError, (hipStream_t)stream, nullptr, kBM, kBM);
+                         ws_ptr<uint32_t>(workspace, L.status) + kStatusError, (hipStream_t)stream, nullptr,
+                         ChunkRows{kBM, kBM, {}, nullptr});
+}
+
+extern "C" int tmoe_debug_prefill_plan(int T, int H, int E, int I, int k, int Is, int q4, int blocks,
+                                       const int32_t* counts, int64_t* plan) {
+  using namespace tmoe;
+  if (!plan) return TMOE_ERR_NULL;
+  if (T < 2 || q4 < 0 || q4 > 2 || blocks < 8 || blocks % 8 || !tmoe_workspace_bytes(T, H, E, I, k, Is) ||
+      H % 128 || I % (q4 ? 128 : 64) || E > 1023 || (Is && Is != I))
+    return TMOE_ERR_SHAPE;
+  const PrefillPlan p = prefill_plan(T, H, E, I, k, Is > 0, q4, false, blocks);
+  int bm = p.bm, bms = p.bms;
+  if (p.rule.lo && counts) {
+    int hit = Is > 0, chunks[3];
+    for (int s = 0; s < 3; ++s) chunks[s] = Is > 0 ? (T + kRowSizes[s] - 1) / kRowSizes[s] : 0;
+    for (int e = 0; e < E; ++e) {
+      hit += counts[e] > 0;
+      for (int s = 0; s < 3; ++s) chunks[s] += (counts[e] + kRowSizes[s] - 1) / kRowSizes[s];
+    }
+    bm = bms = chunk_pick(p.rule, hit, chunks);
+  }
+  const Ws L = ws_layout(T, H, E, I, k, Is);
+  plan[0] = bm;
+  plan[1] = bms;
+  plan[2] = p.fuse;
+  plan[3] = p.tiled;
+  plan[4] = (int64_t)(L.scratch + sizeof(int32_t) * rows_word(E));
+  return TMOE_OK;
 }

@@ -1,0 +1,75 @@
+"""The prefill path's plan (rows per M-chunk), computed on the host: no GPU."""
+import numpy as np
+import pytest
+
+from tarfa_amd._lib import lib
+
+CUS = 256
+
+
+def plan(T, H, E, I, k, Is=0, q4=0, counts=None):
+    out = np.zeros(5, np.int64)
+    c = None if counts is None else np.ascontiguousarray(counts, np.int32)
+    st = lib().tmoe_debug_prefill_plan(T, H, E, I, k, Is, q4, CUS, None if c is None else c.ctypes.data,
+                                       out.ctypes.data)
+    assert st == 0, st
+    return out.tolist()
+
+
+def uniform(T, E, k, seed=0):
+    r = np.random.default_rng(seed)
+    return np.bincount(r.random((T, E)).argpartition(k, axis=1)[:, :k].ravel(), minlength=E)
+
+
+def hot(T, E, k):
+    """Every token takes the same k experts."""
+    return np.where(np.arange(E) < k, T, 0)
+
+
+FULL = (2560, 256, 1024, 8, 1024)
+
+
+@pytest.mark.parametrize("T,routing,rows", [
+    (18, uniform, 32), (18, hot, 32), (40, hot, 64), (211, uniform, 32), (603, uniform, 32), (1024, uniform, 64),
+    (400, hot, 64), (603, hot, 64), (1024, hot, 160), (1536, hot, 160), (2048, uniform, 160), (4096, uniform, 160)])
+def test_bf16_rows_follow_the_group_sizes(T, routing, rows):
+    """Measured at the full-size layer with each size forced: a routing that sends every token to the same
+    experts took 128 us at T = 400 with 160 rows, 152 with the 32 that a uniform routing wants."""
+    H, E, I, k, Is = FULL
+    assert plan(T, H, E, I, k, Is, counts=routing(T, E, k))[:2] == [rows, rows]
+
+
+def test_bf16_rows_few_large_groups():
+    """Few groups leave blocks idle at 160 rows (E = 8 of mean 128 rows: 91 us against 73)."""
+    assert plan(512, 1280, 8, 1920, 2, counts=uniform(512, 8, 2))[0] == 64
+    assert plan(256, 768, 16, 640, 4, 640, counts=uniform(256, 16, 4))[0] == 64
+
+
+def _cost(s, hit, chunks, H, I):
+    first, further, turn = ((285, 90, 100), (300, 100, 112), (320, 200, 230))[s]
+    up, dn = I // 128, H // 256
+    work = (first * hit + further * (chunks - hit)) * (up * H + dn * I)
+    return max(work, turn * CUS * (-(-chunks * up // CUS) * H + -(-chunks * dn // CUS) * I))
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_bf16_rows_are_the_cheapest(seed):
+    """The choice over random group sizes, up to the most entries a call may have, against the cost in
+    Python integers."""
+    r = np.random.default_rng(seed)
+    H, I = 256 * int(r.integers(2, 17)), 128 * int(r.integers(4, 33))
+    E, k = int(r.integers(1, 1024)), 1
+    T = int(np.exp(r.uniform(np.log(20), np.log(524288))))
+    p = r.dirichlet(np.full(E, r.choice([0.02, 0.3, 5.0])))
+    c = r.multinomial(T, p)
+    Is = int(r.choice([0, I]))
+    got, shared, _, tiled, _ = plan(T, H, E, I, k, Is, counts=c)
+    smallest = plan(T, H, E, I, k, Is)[0]
+    assert got == shared
+    if not tiled or smallest == 160:
+        assert got == 160
+        return
+    hit = int((c > 0).sum()) + (Is > 0)
+    costs = {rows: _cost(s, hit, int((-(-c // rows)).sum()) + (-(-T // rows) if Is else 0), H, I)
+             for s, rows in enumerate((32, 64, 160)) if rows >= smallest}
+    assert costs[got] <= min(costs.values()) * (1 + 1e-5)          # the rule is in fp32

@@ -1,6 +1,6 @@
-"""The prefill GEMMs' chunk sizes: groups of 1, 31, 32, 33, 64 and 65 rows through 16- to 64-row chunks
-(the rule takes the fewest rows that hold a mean group plus two standard deviations), at widths that
-take four or five weight stages per cycle, against the oracle's chain at the bf16 bars."""
+"""The prefill GEMMs' chunk sizes: groups at the edges of 16- to 160-row chunks, at widths that take four
+or five weight stages per cycle, against the oracle's chain at the bf16 bars; every case asserts the chunk
+size that it runs."""
 import numpy as np
 import pytest
 import torch
@@ -10,50 +10,75 @@ from tarfa_amd import moe as tm
 from tarfa_amd import seeded
 from tarfa_amd.moe import MoEShape, Workspace
 from tests._util import assert_close_bf16, expert_dicts, f32
+from tests.test_chunk_rows import hot, plan, uniform
 
 pytestmark = pytest.mark.gpu
 
 ROWS = [1, 31, 32, 33, 64, 65]
 
 
-def _ids(E, seed):
-    """One expert per token, expert e taken by ROWS[e] tokens in a shuffled order."""
-    ids = np.repeat(np.arange(len(ROWS)), ROWS)
+def _ids(rows, seed):
+    """One expert per token, expert e taken by rows[e] tokens in a shuffled order."""
+    ids = np.repeat(np.arange(len(rows)), rows)
     np.random.default_rng(seed).shuffle(ids)
     return ids[:, None].astype(np.int64)
 
 
-@pytest.mark.parametrize("H,I,E", [(768, 640, 16), (768, 640, 6), (1280, 512, 16), (512, 768, 6)])
-def test_bf16_chunk_edges(gpu, H, I, E):
-    shape = MoEShape(H, E, I, 1, 0)                # mean 14 rows (E = 16) or 38 (E = 6)
+def _device_rows(shape, T, ws, p):
+    """The rows per chunk that the last call's dispatch chose."""
+    assert shape.ws_bytes(T) <= ws.buf.numel()
+    return int(ws.buf[p[4]:p[4] + 4].cpu().view(torch.int32)[0])
+
+
+EDGES = [1, 31, 32, 33, 63, 64, 65, 128, 129, 159, 160, 161, 320, 321]
+
+
+@pytest.mark.parametrize("H,I,rows,chunk", [
+    (768, 640, ROWS + [0] * 10, 32), (1280, 512, ROWS, 32), (512, 768, ROWS + [0] * 10, 32),
+    (768, 640, EDGES, 64), (1280, 512, EDGES, 64), (512, 768, EDGES, 64),
+    (768, 640, EDGES * 4, 160), (1280, 512, EDGES * 3, 160), (512, 768, EDGES * 4, 160)])
+def test_bf16_chunk_edges(gpu, H, I, rows, chunk):
+    E = len(rows)
+    shape = MoEShape(H, E, I, 1, 0)
     layer = seeded.make_layer(shape, H + E, device=gpu)
-    ids = _ids(E, H)
+    ids = _ids(rows, H)
     T = len(ids)
+    p = plan(T, H, E, I, 1, counts=rows)
+    assert p[0] == chunk
     ws = Workspace(shape, gpu, tokens=T)
     x = seeded.make_tokens(shape, H + E, T, device=gpu)
     w = torch.linspace(0.1, 1.0, T, device=gpu).to(torch.bfloat16)[:, None].contiguous()
     out = tm.experts_forward(shape, x, torch.from_numpy(ids).to(gpu), w, tm.expert_table(layer.gate_up, layer.down),
                              ws)
+    assert _device_rows(shape, T, ws, p) == chunk
     gu, dn = expert_dicts(layer.gate_up, layer.down, ids)
-    assert_close_bf16(f32(out), moe.experts_prefill(f32(x), ids, f32(w), gu, dn, E), f"H={H} I={I} E={E}")
+    assert_close_bf16(f32(out), moe.experts_prefill(f32(x), ids, f32(w), gu, dn, E), f"H={H} I={I} chunk={chunk}")
     ws.status()
 
 
-@pytest.mark.parametrize("T,I", [(17, 768), (90, 768), (200, 768), (4096, 640)])
-def test_bf16_chunks_with_shared_expert(gpu, T, I):
-    """Mean groups of 4, 22, 50 and 1024 rows, the shared expert in the same chunks; the last in 160-row
-    chunks whose down GEMM takes five-stage cycles."""
-    shape = MoEShape(768, 16, I, 4, I)
+@pytest.mark.parametrize("T,I,routing,chunk", [
+    (17, 768, uniform, 32), (90, 768, uniform, 32), (160, 768, uniform, 64), (160, 768, hot, 32),
+    (1000, 768, hot, 64), (2000, 768, uniform, 160), (4096, 640, uniform, 160), (4096, 640, hot, 160)])
+def test_bf16_chunks_with_shared_expert(gpu, T, I, routing, chunk):
+    """The shared expert in the same chunks; a routing that spreads over the experts, and one that sends
+    every token to the same four (group sizes that only the dispatch sees).  I = 640: the 160-row down
+    GEMM's five-stage cycles."""
+    E, k = 16, 4
+    shape = MoEShape(768, E, I, k, I)
     layer = seeded.make_layer(shape, T, device=gpu)
     ws = Workspace(shape, gpu, tokens=T)
     x = seeded.make_tokens(shape, T, T, device=gpu)
     logits = seeded.make_logits(shape, T, T, device=gpu)
+    if routing is hot:
+        logits[:, :k] += 1000.0
     table = tm.expert_table(layer.gate_up, layer.down)
     out, ids, w = tm.moe_block(shape, x, table, ws, logits=logits, shared=layer.shared)
     ids = ids.cpu().numpy()
-    assert np.array_equal(ids, moe.router_topk(logits.cpu().numpy(), 4)[0])
+    assert np.array_equal(ids, moe.router_topk(logits.cpu().numpy(), k)[0])
+    p = plan(T, 768, E, I, k, I, counts=np.bincount(ids.ravel(), minlength=E))
+    assert p[0] == chunk and _device_rows(shape, T, ws, p) == chunk
     gu, dn = expert_dicts(layer.gate_up, layer.down, ids)
-    ref = moe.add_bf16(moe.experts_prefill(f32(x), ids, f32(w), gu, dn, 16),
+    ref = moe.add_bf16(moe.experts_prefill(f32(x), ids, f32(w), gu, dn, E),
                        moe.shared_expert(f32(x), *[f32(t) for t in layer.shared]))
     assert_close_bf16(f32(out), ref, f"T={T}")
     ws.status()
@@ -85,7 +110,7 @@ def test_int4_chunk_edges(gpu, H, I, E, rows):
     shape = MoEShape(H, E, I, 1, 0)
     layer = seeded.make_layer(shape, H + E, device=gpu)
     parts, table, gu, dn = _q4(layer, rows, gpu)
-    ids = _ids(E, H)
+    ids = _ids(ROWS, H)
     T = len(ids)
     ws = Workspace(shape, gpu, tokens=T)
     x = seeded.make_tokens(shape, H + E, T, device=gpu)
