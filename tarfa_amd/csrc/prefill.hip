@@ -2049,6 +2049,7 @@ struct PrefillPlan {
   int bm, bms;                    // rows per chunk, routed and shared (where rule.lo is 0)
   ChunkRule rule;                 // bf16: how the dispatch chooses them
 };
+static size_t logits_desc_entries(int T, int E) { return sizeof(float) * (size_t)T * (E + 1) / sizeof(int4); }
 static PrefillPlan prefill_plan(int T, int H, int E, int I, int k, bool has_sh, int q4, bool frag, int blocks) {
   PrefillPlan p{};
   // A rows are addressed with 32-bit byte offsets by the persistent kernels.
@@ -2063,22 +2064,23 @@ static PrefillPlan prefill_plan(int T, int H, int E, int I, int k, bool has_sh, 
   // Small-group int4 kernel: the same tiles, at least kQB stages of 128.
   const bool qline = I % kPUpCols == 0 && H % kPDnCols == 0 && ofs32 && H / kQK >= kQB && I / kQK >= kQB;
   p.tiled = !frag && (q4 ? qline && (!has_sh || p.line) : p.line);
-  // The smallest chunks the call may use; more of them than the descriptor region holds (T k / 64)
-  // go to the router logits' region, read for the last time by the top-k launch.
+  // The smallest chunks the call may use.  Their descriptors lie in their own region, or, where that
+  // (T k / 64) is too small, in the router logits', read for the last time by the top-k launch; where
+  // neither holds the most that T k entries can make, the chunks are larger.
   int bm = kBM;
   if (p.tiled) bm = q4 ? chunk_rows_q4(T, k, E, p.persistent && H >= 2 * kcyc) : 32;
-  for (; bm != kBM; bm = q4 || bm == 64 ? kBM : 64) {
-    const size_t hit = (size_t)T * k < (size_t)E ? (size_t)T * k : (size_t)E;
-    const size_t chunks = (size_t)T * k / bm + hit + T / (bm < kQShared ? bm : kQShared) + 2;
-    if (16 * chunks <= sizeof(float) * (size_t)T * (E + 1)) break;
+  for (;; bm = q4 || bm == 64 ? kBM : 64) {
+    // Int4 groups in chunks of at most 32 rows: the shared expert runs inside the routed launches, where
+    // its K takes four-stage cycles (with 64-row chunks, whose many shared tiles run as fast by
+    // themselves, it gets launches of its own: T=700 388 us against 409, T=1024 457 against 441).
+    p.fuse = q4 && has_sh && bm <= 32 && I % (4 * kBK) == 0;
+    p.bm = bm;
+    p.bms = p.fuse ? kQShared : q4 && bm != kBM ? 64 : bm;
+    const size_t n = (size_t)T * k, hit = n < (size_t)E ? n : (size_t)E;
+    const size_t chunks = hit + (n - hit) / bm + (has_sh ? (T + p.bms - 1) / p.bms : 0);
+    p.desc_logits = chunks > desc_entries(T, E, k);
+    if (!p.desc_logits || bm == kBM || chunks <= logits_desc_entries(T, E)) break;
   }
-  p.desc_logits = bm != kBM;
-  // Int4 groups in chunks of at most 32 rows: the shared expert runs inside the routed launches, where
-  // its K takes four-stage cycles (with 64-row chunks, whose many shared tiles run as fast by
-  // themselves, it gets launches of its own: T=700 388 us against 409, T=1024 457 against 441).
-  p.fuse = q4 && has_sh && bm <= 32 && I % (4 * kBK) == 0;
-  p.bm = bm;
-  p.bms = p.fuse ? kQShared : q4 && bm != kBM ? 64 : bm;
   if (!q4 && bm != kBM)
     p.rule = ChunkRule{bm, (float)H, (float)I, (float)(I / kPUpCols) / blocks, (float)(H / kPDnCols) / blocks};
   return p;
@@ -2257,5 +2259,6 @@ extern "C" int tmoe_debug_prefill_plan(int T, int H, int E, int I, int k, int Is
   plan[2] = p.fuse;
   plan[3] = p.tiled;
   plan[4] = (int64_t)(L.scratch + sizeof(int32_t) * rows_word(E));
+  plan[5] = (int64_t)(p.desc_logits ? logits_desc_entries(T, E) : desc_entries(T, E, k));
   return TMOE_OK;
 }

@@ -75,14 +75,17 @@ struct Ws {
   size_t inv;      // int32[T * k]
   size_t scratch;  // int32[E + 64]      dispatch counters
   size_t ch;       // bf16[T * k * H]    per-assignment expert outputs, unscaled (T > 1)
-  size_t desc;     // int32x4[T * k / 64 + E + T / 64 + 2]   prefill M-chunk descriptors (T > 1; chunks of
-                   // fewer than 160 rows, more of them, lie in the logits region once the top-k has run)
+  size_t desc;     // int32x4[desc_entries(T, E, k)]   prefill M-chunk descriptors (T > 1; those of small
+                   // chunks, where there can be more, lie in the logits region once the top-k has run)
   size_t xn;       // bf16[T * H]        RMSNorm of the hidden state (the layer entry points)
   size_t sbord;    // small-batch combine order: int32 rows[kSbMaxEntries], f32 weights[kSbMaxEntries],
                    // int32 counts[kSbMaxTokens]; then the down kernel's slice descriptors
                    // (16 bytes each: a header and up to kSbMaxEntries + 2 slices)
   size_t total;
 };
+
+// Room for chunks of 160 rows (and of 64).
+inline size_t desc_entries(size_t T, size_t E, size_t k) { return T * k / 64 + E + T / 64 + 2; }
 
 inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
@@ -106,7 +109,7 @@ inline Ws ws_layout(int T, int H, int E, int I, int k, int Is) {
   w.inv = take(sizeof(int32_t) * t * (size_t)k);
   w.scratch = take(sizeof(int32_t) * (size_t)(E + 64));
   w.ch = take(t > 1 ? 2 * t * (size_t)k * (size_t)H : 0);
-  w.desc = take(t > 1 ? 16 * (t * (size_t)k / 64 + (size_t)E + t / 64 + 2) : 0);
+  w.desc = take(t > 1 ? 16 * desc_entries(t, E, k) : 0);
   w.xn = take(2 * t * (size_t)H);
   w.sbord = take(4 * (2 * (size_t)kSbMaxEntries + kSbMaxTokens) + 16 * ((size_t)kSbMaxEntries + 3));
   w.total = o;

@@ -8,7 +8,7 @@ CUS = 256
 
 
 def plan(T, H, E, I, k, Is=0, q4=0, counts=None):
-    out = np.zeros(5, np.int64)
+    out = np.zeros(6, np.int64)
     c = None if counts is None else np.ascontiguousarray(counts, np.int32)
     st = lib().tmoe_debug_prefill_plan(T, H, E, I, k, Is, q4, CUS, None if c is None else c.ctypes.data,
                                        out.ctypes.data)
@@ -63,7 +63,7 @@ def test_bf16_rows_are_the_cheapest(seed):
     p = r.dirichlet(np.full(E, r.choice([0.02, 0.3, 5.0])))
     c = r.multinomial(T, p)
     Is = int(r.choice([0, I]))
-    got, shared, _, tiled, _ = plan(T, H, E, I, k, Is, counts=c)
+    got, shared, _, tiled = plan(T, H, E, I, k, Is, counts=c)[:4]
     smallest = plan(T, H, E, I, k, Is)[0]
     assert got == shared
     if not tiled or smallest == 160:
@@ -73,3 +73,36 @@ def test_bf16_rows_are_the_cheapest(seed):
     costs = {rows: _cost(s, hit, int((-(-c // rows)).sum()) + (-(-T // rows) if Is else 0), H, I)
              for s, rows in enumerate((32, 64, 160)) if rows >= smallest}
     assert costs[got] <= min(costs.values()) * (1 + 1e-5)          # the rule is in fp32
+
+
+@pytest.mark.parametrize("E,k,Is", [(32, 8, 1024), (16, 4, 512), (16, 6, 512), (16, 8, 0), (256, 8, 1024), (8, 2, 512),
+                                    (1, 1, 512)])
+@pytest.mark.parametrize("q4", [0, 1, 2])
+def test_small_calls_take_small_chunks(E, k, Is, q4):
+    """Few tokens leave few logits; their descriptors fit the region of their own (int4 E = 32, k = 8,
+    T = 2 .. 4 ran 160-row tiles: 151 us against 84 at T = 5, H = 2560, I = 640)."""
+    I = Is or 512
+    for T in range(2, 6):
+        rows, shared, fuse, tiled = plan(T, 1024, E, I, k, Is, q4)[:4]
+        assert tiled and (rows == 16 if q4 else rows == 32)
+        assert fuse == (q4 > 0 and Is > 0) and shared == (32 if fuse or not q4 else 64)
+
+
+@pytest.mark.parametrize("seed", range(30))
+def test_descriptors_fit_their_region(seed):
+    """The most chunks that T k entries can make: every expert one row, the rest on one of them."""
+    r = np.random.default_rng(seed)
+    E = int(np.exp(r.uniform(0, np.log(1023.9))))
+    k = int(r.integers(1, min(E, 16) + 1))
+    Is = int(r.choice([0, 768]))
+    for T in sorted({2, 3, *np.exp(r.uniform(np.log(2), np.log((1 << 19) / k), 20)).astype(int).tolist()}):
+        for q4 in (0, 1):
+            rows, shared, _, _, _, room = plan(T, 1024, E, 768, k, Is, q4)
+            hit = min(T * k, E)
+            spread = np.full(hit, (T * k) // hit)
+            spread[0] += T * k - spread.sum()
+            one = np.ones(hit, int)
+            one[0] = T * k - hit + 1                   # past T: more than distinct experts per token allow
+            for c in (spread, one):
+                chunks = int((-(-c // rows)).sum()) + (-(-T // shared) if Is else 0)
+                assert chunks <= room, (T, E, k, Is, q4, rows)

@@ -108,6 +108,7 @@ def _q4(layer, rows, gpu):
 def test_int4_chunk_edges(gpu, H, I, E, rows):
     """Means of 6, 14 and 38 rows: 16-, 32- and 64-row chunks; K of 4 (the fewest), 5 and 6 stages."""
     shape = MoEShape(H, E, I, 1, 0)
+    assert plan(sum(ROWS), H, E, I, 1, q4=1 + rows)[0] == {40: 16, 16: 32, 6: 64}[E]
     layer = seeded.make_layer(shape, H + E, device=gpu)
     parts, table, gu, dn = _q4(layer, rows, gpu)
     ids = _ids(ROWS, H)
@@ -121,11 +122,13 @@ def test_int4_chunk_edges(gpu, H, I, E, rows):
 
 
 @pytest.mark.parametrize("rows", [False, True])
-@pytest.mark.parametrize("T,I", [(2, 512), (33, 512), (90, 512), (200, 512), (33, 640), (900, 640)])
-def test_int4_chunks_with_shared_expert(gpu, T, I, rows):
+@pytest.mark.parametrize("T,I,chunk,fuse", [(2, 512, 16, 1), (4, 768, 16, 1), (33, 512, 16, 1), (90, 512, 32, 1),
+                                            (200, 512, 64, 0), (33, 640, 16, 0), (900, 640, 64, 0)])
+def test_int4_chunks_with_shared_expert(gpu, T, I, chunk, fuse, rows):
     """Mean groups of 0.5 to 225 rows; the shared expert's tiles inside the int4 launches (I = 512, up to
     32-row chunks) or in launches of their own."""
     shape = MoEShape(768, 16, I, 4, I)
+    assert plan(T, 768, 16, I, 4, I, q4=1 + rows)[:4] == [chunk, 32 if fuse else 64, fuse, 1]
     layer = seeded.make_layer(shape, T, device=gpu)
     parts, table, gu, dn = _q4(layer, rows, gpu)
     ws = Workspace(shape, gpu, tokens=T)
