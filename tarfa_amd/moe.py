@@ -35,6 +35,9 @@ def _p(t):
 
 def _stream(device):
     # The current stream's handle without building a torch.cuda.Stream object (~4 us of host time a call).
+    # Host memory is refused here, as that object's lookup would: some callers check nothing else.
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 

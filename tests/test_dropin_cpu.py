@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from tarfa_amd import experts as tx
+from tarfa_amd.residency import RouteTelemetry
 
 
 def _tf_block(dtype):
@@ -36,3 +37,12 @@ def test_forward_rejects_a_non_bf16_hidden_state():
     with pytest.raises(TypeError, match="bfloat16"):
         fwd(None, torch.zeros(1, 64, dtype=torch.float16), torch.zeros(1, 2, dtype=torch.int64),
             torch.zeros(1, 2))
+
+
+def test_route_telemetry_refuses_host_ids():
+    """Before a launch: the kernel would read them as device memory."""
+    t = RouteTelemetry(1, 8, 32, device="cpu")
+    with pytest.raises(ValueError, match="cuda device"):
+        t.record(torch.zeros(1, 8, dtype=torch.int64))
+    with pytest.raises(ValueError, match="cuda device"):
+        t.record()
