@@ -63,14 +63,23 @@ class Workspace:
 
     def __init__(self, shape: MoEShape, device, tokens=1):
         self.shape, self.device = shape, torch.device(device)
-        self.buf = None
+        self._buf = self.status_word = None
         self.ensure(tokens)
+
+    @property
+    def buf(self):
+        return self._buf
+
+    @buf.setter
+    def buf(self, buf):
+        # status_word: the view that decode calls copy, made once per buffer (~3 us of host time a call).
+        self._buf = buf
+        self.status_word = None if buf is None else buf[:4].view(torch.int32)
 
     def ensure(self, tokens):
         need = self.shape.ws_bytes(tokens)
         if self.buf is None or self.buf.numel() < need:
             self.buf = torch.zeros(need, dtype=torch.uint8, device=self.device)
-            self.status_word = self.buf[:4].view(torch.int32)
         return self.buf
 
     def status(self):

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from tarfa_amd import experts as tx
+from tarfa_amd.moe import MoEShape, Workspace
 from tarfa_amd.residency import RouteTelemetry
 
 
@@ -46,3 +47,15 @@ def test_route_telemetry_refuses_host_ids():
         t.record(torch.zeros(1, 8, dtype=torch.int64))
     with pytest.raises(ValueError, match="cuda device"):
         t.record()
+
+
+def test_workspace_status_word_follows_its_buffer():
+    """Workspaces may share one buffer, and grow: the polled word is always the current buffer's."""
+    shape = MoEShape(64, 4, 32, 2)
+    a, b = Workspace(shape, "cpu"), Workspace(shape, "cpu")
+    b.buf = a.buf
+    assert b.status_word.data_ptr() == a.buf.data_ptr()
+    a.buf[0] = 1
+    assert int(b.status_word[0]) == 1
+    b.ensure(64)
+    assert b.status_word.data_ptr() == b.buf.data_ptr() != a.buf.data_ptr()
