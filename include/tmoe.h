@@ -294,7 +294,8 @@ int tmoe_debug_decode_trace(void* buf, size_t bytes);
  * plan[0], plan[1]: rows per M-chunk, routed experts and shared expert; plan[2]: 1 where the shared
  * expert runs inside the int4 launches; plan[3]: 1 where the whole-line bf16 and small-group int4
  * kernels take the shape; plan[4]: the workspace byte where a call leaves the bf16 GEMMs' rows per
- * chunk (int32); plan[5]: the M-chunks that the region of their descriptors holds.
+ * chunk (int32); plan[5]: the M-chunks that the region of their descriptors holds; plan[6],
+ * plan[7]: tokens and experts per tile of the router logits (T >= 128).
  */
 int tmoe_debug_prefill_plan(int T, int H, int E, int I, int k, int Is, int q4, int blocks,
                             const int32_t* counts, int64_t* plan);

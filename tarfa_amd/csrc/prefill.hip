@@ -2041,6 +2041,8 @@ static void gemm_q_launch(const GemmParams& g, int bm, unsigned grid, hipStream_
   else hipLaunchKernelGGL((k_grouped_gemm_q<UP, QR, 4>), gd, bd, 0, s, g);
 }
 
+void router_tile(int T, int E, int cus, int* ta, int* tb);   // router.hip
+
 // What a prefill call of this shape launches; host arithmetic only.
 struct PrefillPlan {
   bool persistent, line, tiled;   // shapes the fragment-load and the whole-line kernel (and k_grouped_gemm_q) take
@@ -2114,12 +2116,9 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
     const char* e = getenv("TMOE_PREFILL_GEMM");
     return e && !strcmp(e, "frag");
   }();
-  static int n_cu[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return TMOE_ERR_HIP;
-  if (!n_cu[dev] && hipDeviceGetAttribute(&n_cu[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return TMOE_ERR_HIP;
-  const unsigned pgrid = (unsigned)(n_cu[dev] >= 8 ? n_cu[dev] / 8 * 8 : 8);
+  const int cus = compute_units();
+  if (!cus) return TMOE_ERR_HIP;
+  const unsigned pgrid = (unsigned)(cus >= 8 ? cus / 8 * 8 : 8);
   const PrefillPlan pl = prefill_plan(T, H, E, I, k, has_sh, q4, frag, (int)pgrid);
   const bool persistent = pl.persistent, line = pl.line, fuse = pl.fuse;
   const int bm = pl.bm, kcyc = kBK * kPR;
@@ -2260,5 +2259,9 @@ extern "C" int tmoe_debug_prefill_plan(int T, int H, int E, int I, int k, int Is
   plan[3] = p.tiled;
   plan[4] = (int64_t)(L.scratch + sizeof(int32_t) * rows_word(E));
   plan[5] = (int64_t)(p.desc_logits ? logits_desc_entries(T, E) : desc_entries(T, E, k));
+  int ta = 0, tb = 0;
+  router_tile(T, E, blocks, &ta, &tb);
+  plan[6] = 16 * ta;
+  plan[7] = 16 * tb;
   return TMOE_OK;
 }

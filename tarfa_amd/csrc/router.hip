@@ -135,6 +135,24 @@ __global__ __launch_bounds__(256) void k_router_topk(const float* __restrict__ l
   wave_topk<MAXEPL>(logits + (size_t)t * E, false, E, k, lane, o);
 }
 
+// Tiles of 16 ta tokens x 16 tb experts: 4 x 4 or 4 x 2 where at least a block per CU remains and its
+// rounds of blocks cost less (a round of 2 x 2, 4 x 2, 4 x 4: about 100, 165, 240), else 2 x 2.  Router
+// call at H=2560, 2 x 2 / 4 x 2 / 4 x 4, us: E=256 T=2048 24.7 / 20.8 / -, T=4096 43.8 / - / 29.9; E=160
+// T=4096 (640 / 320 / 192 blocks) 34.8 / 34.7 / 28.3, at H=1024 19.0 / 19.3 / 16.8.  Up to 16 experts a
+// wider tile is padding (E=8 T=16384 28.5 / 30.2 / 31.9).
+void router_tile(int T, int E, int cus, int* ta, int* tb) {
+  constexpr int A[3] = {2, 4, 4}, B[3] = {2, 2, 4}, turn[3] = {100, 165, 240};
+  long least = 0;
+  for (int i = 0; i < 3; ++i) {
+    const long blocks = (long)((T + 16 * A[i] - 1) / (16 * A[i])) * ((E + 16 * B[i] - 1) / (16 * B[i]));
+    const long cost = (blocks + cus - 1) / cus * turn[i];
+    if (i && (E <= 16 || blocks < cus || cost >= least)) continue;
+    least = cost;
+    *ta = A[i];
+    *tb = B[i];
+  }
+}
+
 int launch_router_logits(const uint16_t* x, const uint16_t* wg, int T, int H, int E, float* logits,
                          hipStream_t s) {
   static const int mfma_from = [] {
@@ -142,15 +160,17 @@ int launch_router_logits(const uint16_t* x, const uint16_t* wg, int T, int H, in
     return e ? atoi(e) : kRouterMfmaFrom;
   }();
   if (T >= mfma_from && H % 32 == 0) {
-    // The largest tile that still leaves a block for each of 256 CUs.
-    auto blocks = [&](int ta, int tb) { return ((T + 16 * ta - 1) / (16 * ta)) * ((E + 16 * tb - 1) / (16 * tb)); };
-    auto grid = [&](int ta, int tb) { return dim3((T + 16 * ta - 1) / (16 * ta), (E + 16 * tb - 1) / (16 * tb)); };
-    if (blocks(4, 4) >= 256)
-      hipLaunchKernelGGL((k_router_logits_mfma<4, 4>), grid(4, 4), dim3(256), 0, s, x, wg, T, H, E, logits);
-    else if (blocks(4, 2) >= 256)
-      hipLaunchKernelGGL((k_router_logits_mfma<4, 2>), grid(4, 2), dim3(256), 0, s, x, wg, T, H, E, logits);
+    const int cus = compute_units();
+    if (!cus) return TMOE_ERR_HIP;
+    int ta, tb;
+    router_tile(T, E, cus, &ta, &tb);
+    const dim3 g((T + 16 * ta - 1) / (16 * ta), (E + 16 * tb - 1) / (16 * tb));
+    if (tb == 4)
+      hipLaunchKernelGGL((k_router_logits_mfma<4, 4>), g, dim3(256), 0, s, x, wg, T, H, E, logits);
+    else if (ta == 4)
+      hipLaunchKernelGGL((k_router_logits_mfma<4, 2>), g, dim3(256), 0, s, x, wg, T, H, E, logits);
     else
-      hipLaunchKernelGGL((k_router_logits_mfma<2, 2>), grid(2, 2), dim3(256), 0, s, x, wg, T, H, E, logits);
+      hipLaunchKernelGGL((k_router_logits_mfma<2, 2>), g, dim3(256), 0, s, x, wg, T, H, E, logits);
     return hipGetLastError() == hipSuccess ? TMOE_OK : TMOE_ERR_HIP;
   }
   const int nc = (H + 511) / 512;

@@ -8,9 +8,22 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "tmoe.h"
 
 namespace tmoe {
+
+// The current device's compute units, asked once per device; 0 where HIP fails.
+inline int compute_units() {
+  static std::atomic<int> known[64];
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if ((n = known[dev].load(std::memory_order_relaxed))) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  known[dev].store(n, std::memory_order_relaxed);
+  return n;
+}
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));

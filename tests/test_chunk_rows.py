@@ -8,7 +8,7 @@ CUS = 256
 
 
 def plan(T, H, E, I, k, Is=0, q4=0, counts=None):
-    out = np.zeros(6, np.int64)
+    out = np.zeros(8, np.int64)
     c = None if counts is None else np.ascontiguousarray(counts, np.int32)
     st = lib().tmoe_debug_prefill_plan(T, H, E, I, k, Is, q4, CUS, None if c is None else c.ctypes.data,
                                        out.ctypes.data)
@@ -97,7 +97,7 @@ def test_descriptors_fit_their_region(seed):
     Is = int(r.choice([0, 768]))
     for T in sorted({2, 3, *np.exp(r.uniform(np.log(2), np.log((1 << 19) / k), 20)).astype(int).tolist()}):
         for q4 in (0, 1):
-            rows, shared, _, _, _, room = plan(T, 1024, E, 768, k, Is, q4)
+            rows, shared, _, _, _, room = plan(T, 1024, E, 768, k, Is, q4)[:6]
             hit = min(T * k, E)
             spread = np.full(hit, (T * k) // hit)
             spread[0] += T * k - spread.sum()
@@ -106,3 +106,12 @@ def test_descriptors_fit_their_region(seed):
             for c in (spread, one):
                 chunks = int((-(-c // rows)).sum()) + (-(-T // shared) if Is else 0)
                 assert chunks <= room, (T, E, k, Is, q4, rows)
+
+
+@pytest.mark.parametrize("T,E,tile", [
+    (4096, 256, [64, 64]), (2048, 256, [64, 32]), (1024, 256, [32, 32]), (16384, 256, [64, 64]),
+    (4096, 160, [32, 32]), (16384, 8, [32, 32]), (16384, 16, [32, 32]), (16384, 32, [64, 32]), (128, 1023, [32, 32])])
+def test_router_tiles(T, E, tile):
+    """Wider tiles only where they fill the chip in fewer or cheaper rounds: E = 160, T = 4096 in 320 blocks and
+    E = 8 in 64-wide tiles were slower than the 32 x 32 tiles they replaced (2 % and 11 %)."""
+    assert plan(T, 2560, E, 512, min(8, E))[6:8] == tile
