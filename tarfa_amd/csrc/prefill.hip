@@ -47,17 +47,20 @@ __device__ __forceinline__ bool ids_aligned(const int32_t* ids32, const int64_t*
 // The dispatch chooses the rows per chunk of the bf16 GEMMs (32, 64 or 160; one size for all groups)
 // from the group sizes, which the host does not know.  A smaller chunk stages and multiplies less
 // padding; a group cut into more of them has its weights read (from L2 or the infinity cache) and
-// staged more often.  In units of 1/100 of the time in which every block multiplies one 32-row tile:
-//   a group's first chunk    285  300  320   (32, 64, 160 rows; its weights come from HBM)
-//   each further one          90  100  200
-//   but a round of tiles     100  112  230   and tiles take whole rounds of the launch's blocks.
-// Fitted to us per call with the size forced, 120 runs of 8 shapes, T = 17 .. 4096, uniform, Zipf and
-// one-set-of-experts routings.  At H=2560 E=256 I=1024 k=8, 32 / 64 / 160 rows:
+// staged more often.  In units of 1/100 of the time in which every block multiplies one 32-row tile
+// (32, 64, 160 rows):
+//   a group's first chunk    305  308  325   (its weights come from HBM)
+//   each further one          91  107  197
+//   a round of tiles         100  114  241   which a launch takes at least, in whole rounds of its
+//                                            blocks; blocks idle in the last one cost 0.63 of that.
+// Fitted to us per call with the size forced, 644 runs (216 shapes, H = 512 .. 4096, I = 512 .. 2048, E =
+// 2 .. 384, T = 17 .. 5595) under uniform, Zipf and one-set-of-experts routings.  At H=2560 E=256 I=1024
+// k=8, 32 / 64 / 160 rows:
 //   T=603  uniform 751 /  758 / 793   Zipf  774 / 768 / 791   every token the same experts 214 / 159 / 182
 //   T=1024         874 /  780 / 817         908 / 817 / 827                                320 / 228 / 216
 //   T=2048        1162 /  932 / 871        1170 / 968 / 957                                599 / 409 / 369
-// The size it names is within 0.3 % of the fastest one on average, 5.4 % at most, and within 0.3 % of 160
-// rows or faster but for two cases (1.5 %: 257 us against 254).
+// The size it names is within 0.3 % of the fastest one on average (10.6 % at most), and slower than 160
+// rows by more than 1 % in four of the runs (4.3 % at most).
 struct ChunkRule {
   int lo = 0;                       // smallest size to choose among (32 or 64; 0: the size is given)
   float H, I;                       // K of the up and of the down launch
@@ -66,13 +69,14 @@ struct ChunkRule {
 constexpr int kRowSizes[3] = {32, 64, kBM};
 // The size to take, where `hit` groups have rows and n[s] chunks of size s hold them.
 __host__ __device__ inline int chunk_pick(const ChunkRule& r, int hit, const int (&n)[3]) {
-  constexpr float first[3] = {285.f, 300.f, 320.f}, further[3] = {90.f, 100.f, 200.f}, turn[3] = {100.f, 112.f, 230.f};
+  constexpr float first[3] = {305.f, 308.f, 325.f}, further[3] = {91.f, 107.f, 197.f}, turn[3] = {100.f, 114.f, 241.f};
+  const float unit = r.up_rounds * r.H + r.dn_rounds * r.I;
   float cost[3];
   for (int s = 0; s < 3; ++s) {
-    const float work = (first[s] * (float)hit + further[s] * (float)(n[s] - hit)) *
-                       (r.up_rounds * r.H + r.dn_rounds * r.I);
-    const float rounds = turn[s] * (ceilf((float)n[s] * r.up_rounds) * r.H + ceilf((float)n[s] * r.dn_rounds) * r.I);
-    cost[s] = work > rounds ? work : rounds;
+    const float whole = ceilf((float)n[s] * r.up_rounds) * r.H + ceilf((float)n[s] * r.dn_rounds) * r.I;
+    const float work = (first[s] * (float)hit + further[s] * (float)(n[s] - hit)) * unit +
+                       0.63f * turn[s] * (whole - (float)n[s] * unit);
+    cost[s] = work > turn[s] * whole ? work : turn[s] * whole;
   }
   return r.lo == 32 && cost[0] <= cost[1] && cost[0] <= cost[2] ? 32 : cost[1] <= cost[2] ? 64 : kBM;
 }

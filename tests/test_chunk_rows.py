@@ -42,20 +42,23 @@ def test_bf16_rows_follow_the_group_sizes(T, routing, rows):
 def test_bf16_rows_few_large_groups():
     """Few groups leave blocks idle at 160 rows (E = 8 of mean 128 rows: 91 us against 73)."""
     assert plan(512, 1280, 8, 1920, 2, counts=uniform(512, 8, 2))[0] == 64
-    assert plan(256, 768, 16, 640, 4, 640, counts=uniform(256, 16, 4))[0] == 64
+    assert plan(256, 768, 16, 640, 4, 640, counts=uniform(256, 16, 4))[0] in (32, 64)
+    assert plan(565, 2048, 14, 1536, 1, 1536, counts=uniform(565, 14, 1))[0] == 160   # one round: 104 us, 64 rows 112
 
 
 def _cost(s, hit, chunks, H, I):
-    first, further, turn = ((285, 90, 100), (300, 100, 112), (320, 200, 230))[s]
+    first, further, turn = ((305, 91, 100), (308, 107, 114), (325, 197, 241))[s]
     up, dn = I // 128, H // 256
-    work = (first * hit + further * (chunks - hit)) * (up * H + dn * I)
-    return max(work, turn * CUS * (-(-chunks * up // CUS) * H + -(-chunks * dn // CUS) * I))
+    whole = CUS * (-(-chunks * up // CUS) * H + -(-chunks * dn // CUS) * I)
+    unit = up * H + dn * I
+    work = (first * hit + further * (chunks - hit)) * unit + 0.63 * turn * (whole - chunks * unit)
+    return max(work, turn * whole)
 
 
 @pytest.mark.parametrize("seed", range(40))
 def test_bf16_rows_are_the_cheapest(seed):
     """The choice over random group sizes, up to the most entries a call may have, against the cost in
-    Python integers."""
+    Python."""
     r = np.random.default_rng(seed)
     H, I = 256 * int(r.integers(2, 17)), 128 * int(r.integers(4, 33))
     E, k = int(r.integers(1, 1024)), 1

@@ -57,7 +57,7 @@ def test_bf16_chunk_edges(gpu, H, I, rows, chunk):
 
 
 @pytest.mark.parametrize("T,I,routing,chunk", [
-    (17, 768, uniform, 32), (90, 768, uniform, 32), (160, 768, uniform, 64), (160, 768, hot, 32),
+    (17, 768, uniform, 32), (90, 768, uniform, 32), (300, 768, uniform, 64), (160, 768, hot, 32),
     (1000, 768, hot, 64), (2000, 768, uniform, 160), (4096, 640, uniform, 160), (4096, 640, hot, 160)])
 def test_bf16_chunks_with_shared_expert(gpu, T, I, routing, chunk):
     """The shared expert in the same chunks; a routing that spreads over the experts, and one that sends
