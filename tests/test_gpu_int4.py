@@ -20,6 +20,7 @@ from tarfa_amd import seeded
 from tarfa_amd import moe as tm
 from tarfa_amd.moe import MoEShape, Workspace
 from tests._util import assert_close_any_bf16, assert_close_bf16, f32
+from tests.test_chunk_rows import plan
 
 pytestmark = pytest.mark.gpu
 
@@ -244,14 +245,16 @@ def test_int4_prefill_matches_dequantised_bf16_chain(gpu, T, shared, I):
     ws.status()
 
 
-@pytest.mark.parametrize("mode", ["int4", "bf16"])
-def test_prefill_one_cycle_tiles(gpu, mode):
-    """H = I = 512: each up-GEMM tile is a single 8-stage cycle (int4: the register-staged
-    kernel takes it; bf16: the whole-line kernel's shortest K, two 4-stage cycles), and at
-    T = 4096 over 16 experts (208 M-chunks) every persistent block walks several tiles, so a
-    tile's successor is prepared within its own cycles; the outputs against the oracle's chain
-    (int4: on the dequantised weights)."""
-    shape = MoEShape(512, 16, 512, 8, 0)
+@pytest.mark.parametrize("mode,H,I,rows,tiled", [
+    ("bf16", 512, 512, 160, 1),       # whole-line kernel: its shortest K, two 4-stage cycles
+    ("int4", 512, 512, 64, 1),        # small-group kernel: its fewest stages, four
+    ("int4", 1024, 512, 160, 1),      # fragment-load kernel: down tiles of a single 8-stage cycle
+    ("int4", 640, 384, 160, 0)])      # register-staged kernel (K no multiple of 256)
+def test_prefill_one_cycle_tiles(gpu, mode, H, I, rows, tiled):
+    """The shortest K of each prefill GEMM.  At T = 4096 over 16 experts (208 to 528 M-chunks) every
+    persistent block walks several tiles, so a tile's successor is prepared within its own few stages; the
+    outputs against the oracle's chain (int4: on the dequantised weights)."""
+    shape = MoEShape(H, 16, I, 8, 0)
     T = 4096
     layer = seeded.make_layer(shape, 77, device=gpu)
     if mode == "int4":
@@ -268,6 +271,8 @@ def test_prefill_one_cycle_tiles(gpu, mode):
     x = seeded.make_tokens(shape, 77, T, device=gpu)
     out, ids, w = tm.moe_block(shape, x, table, ws, router_w=layer.router_w)
     torch.cuda.synchronize()
+    counts = np.bincount(ids.cpu().numpy().ravel(), minlength=16)
+    assert plan(T, H, 16, I, 8, q4=int(mode == "int4"), counts=counts)[:4] == [rows, rows, 0, tiled]
     ref = moe.experts_prefill(f32(x), ids.cpu().numpy(), f32(w), gu, dn, shape.num_experts)
-    assert_close_bf16(f32(out), ref, f"{mode} prefill H=512 T=4096")
+    assert_close_bf16(f32(out), ref, f"{mode} prefill H={H} T=4096")
     ws.status()
