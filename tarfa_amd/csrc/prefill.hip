@@ -1186,7 +1186,7 @@ __global__ __launch_bounds__(64 * kPW, 1) void k_grouped_gemm_p(GemmParams p) {
 //   A: as in k_grouped_gemm_p (direct global -> LDS loads of whole rows), in a ring of kWAS
 //   slots requested kWA stages ahead; the slot is a run-time index (stage % kWAS).
 // Iteration g: request A stage g + kWA; wait for weight stage g; its registers to the region;
-// request weight stage g + kWB into them; 40 MFMAs; wait for A stage g + 1; barrier.
+// request weight stage g + kWB into them; 4 MB MFMAs; wait for A stage g + 1; barrier.
 // K: a multiple of WB stages and at least 2 WB (the next tile's perm words, requested
 // after a tile's epilogue, are used before its last cycle, WB stage waits later).
 // MB: 16-row token blocks per tile (10: 160-row chunks; 4 and 2 for smaller groups, whose padding
@@ -2137,7 +2137,7 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
   // One GEMM over groups [lo, hi): bf16 weights, or int4 routed weights (the shared
   // group, always bf16, then gets a launch of its own).
   // bf16 groups run on the whole-line kernel where it takes the shape; TMOE_PREFILL_GEMM=frag
-  // selects the fragment-load kernel (int4 groups always use it).
+  // selects the fragment-load kernel, which int4 groups in 160-row chunks always use.
   auto gemm = [&](GemmParams g, int lo, int hi, bool routed_q4, long mchunks) {
     g.group_lo = lo;
     g.group_hi = hi;
@@ -2183,11 +2183,11 @@ int prefill_launch(const uint16_t* x, int T, const int32_t* ids32, const int64_t
   dn.shw0 = sh_down; dn.shw1 = nullptr; dn.out = ch; dn.out_sh = sh;
   if (q4) {
     if (fuse) {
-      const float sh = (float)((T + kQShared - 1) / kQShared);
+      const float tiles = (float)((T + kQShared - 1) / kQShared);
       const float hit = (float)E * (1.0f - powf(1.0f - (float)k / (float)E, (float)T));
       // Blocks in proportion to the tiles, a shared one (four times the weight bytes) counted as two:
       // T=256 383 / 346 / 345 / 351 / 370 us counted as 1 / 2 / 3 / 4 / 6, T=400 382 / 363 / 384 / 388 / 404.
-      const int nb = (int)(4.0f * (float)pgrid * sh / (2.0f * sh + hit) + 7.0f) / 8 * 8;
+      const int nb = (int)(4.0f * (float)pgrid * tiles / (2.0f * tiles + hit) + 7.0f) / 8 * 8;
       up.sh_blocks = dn.sh_blocks = nb < 8 ? 8 : nb > (int)pgrid ? (int)pgrid : nb;
     }
     gemm(up, 0, E, true, mbound);

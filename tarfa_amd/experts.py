@@ -80,9 +80,11 @@ class _CallBook:
             self._raise_if_flagged(int(self._status_host[0]))
         total = self.counts["decode"] + self.counts["prefill"]
         if self.status_poll > 0 and self._status_event is None and total % self.status_poll == 0:
-            # Decode calls copy the word on their own stream: a 1.5 us copy there, where the fork to a
-            # side stream (a wait, an event, a stream switch) took half of a small decode call's ~79 us
-            # of host time.  Longer calls keep it off the compute stream.
+            # Decode calls copy the word on their own stream, where the fork to a side stream (a wait, an
+            # event, a stream switch) took half of a decode call's ~80 us of host time.  us per call, side
+            # stream -> own: H=1024 E=32 I=512 84 -> 29-38, H=2560 E=256 I=1024 80 -> 36; queued behind
+            # other work, where only the GPU's time counts, 21.5 / 34.9 both ways.  Longer calls keep the
+            # copy off the compute stream.
             if inline:
                 self._status_host.copy_(self.workspace.status_word, non_blocking=True)
                 self._inline_event.record(stream)
