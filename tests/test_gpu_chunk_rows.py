@@ -158,3 +158,36 @@ def test_dispatch_one_launch_bounds(gpu, T, E, k):
     inv_ref[p_ref] = np.arange(n)
     assert np.array_equal(inv.cpu().numpy(), inv_ref)
     ws.status()
+
+
+def test_captured_call_follows_each_replays_routing(gpu):
+    """One captured call, replayed on routings that want other chunk sizes (160, 64 and 32 rows), with eager
+    calls between: each replay's bits are the eager call's."""
+    E, k, T = 16, 4, 2400
+    shape = MoEShape(768, E, 768, k, 0)
+    layer = seeded.make_layer(shape, T, device=gpu)
+    ws = Workspace(shape, gpu, tokens=T)
+    x = seeded.make_tokens(shape, T, T, device=gpu)
+    table = tm.expert_table(layer.gate_up, layer.down)
+    slots = torch.arange(k, device=gpu)
+    spread = (torch.arange(T, device=gpu)[:, None] * 5 + slots * 4) % E
+    one = slots.repeat(T, 1)
+    few = torch.full((T, k), E, dtype=torch.int64, device=gpu)       # 40 tokens routed, the rest skipped
+    few[:40] = spread[:40]
+    w = torch.full((T, k), 0.25, dtype=torch.bfloat16, device=gpu)
+    ids = spread.clone()
+    tm.experts_forward(shape, x, ids, w, table, ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = tm.experts_forward(shape, x, ids, w, table, ws)
+    for routing, rows in ((spread, 160), (one, 64), (few, 32), (spread, 160), (few, 32), (one, 64)):
+        want = tm.experts_forward(shape, x, routing, w, table, ws).clone()
+        torch.cuda.synchronize()
+        ids.copy_(routing)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        p = plan(T, 768, E, 768, k, counts=np.bincount(routing.cpu().numpy().ravel(), minlength=E + 1)[:E])
+        assert p[0] == rows and _device_rows(shape, T, ws, p) == rows
+    ws.status()
