@@ -154,7 +154,7 @@ def test_checker_flags_a_copy_before_the_wait():
     assert early_uses(other) == []                     # past an unconditional branch: no path leads there
 
 
-def test_checker_follows_branches_and_back_edges():
+def test_walk_follows_branches_and_back_edges():
     load = "global_load_dwordx4 v[8:11], v1, s[0:1]"
     # A loop whose load is read one trip later; the wait at its head covers it, or does not.
     loop = [".LBB0_1:", "s_waitcnt vmcnt({})", "v_mov_b32_e32 v3, v8", load, "global_store_dword v1, v2, s[0:1]",
@@ -170,7 +170,7 @@ def test_checker_follows_branches_and_back_edges():
     assert early_uses(again) == [(load, load)]
 
 
-def test_checker_path_facts():
+def test_walk_heeds_path_facts():
     load = "global_load_dword v8, v1, s[0:1]"
     # Two stores between the load and its wait: a fact about the loop's trips rules the one-trip path out.
     body = [load, ".LBB0_1:", "; path + store", "global_store_dword v1, v2, s[0:1]", "s_cbranch_scc1 .LBB0_1",
